@@ -143,9 +143,8 @@ struct GemmSpec {
   int64_t ld_aux;
 };
 
-// x then y, in one launch where both GEMMs are of a shape that leaves half
-// of the chip's block slots empty (gemm_f32.hip); otherwise one after the
-// other.  The two must be independent: neither reads what the other writes.
+// x then y, in one launch where both GEMMs take the same large tile shape
+// (gemm_f32.hip); otherwise one after the other.  The two must be independent: neither reads what the other writes.
 // With cs_out set, also cs_out[c] (+)= the sum of column c of the
 // column-major [cs_rows, cs_cols] cs_in (a bias gradient), in the launch of
 // y's split-K reduce when there is one (the same bits as column_sum).
@@ -153,9 +152,10 @@ int gemm_f32_pair(const GemmSpec& x, const GemmSpec& y, hipStream_t st, const ch
                   const float* cs_in = nullptr, float* cs_out = nullptr, int64_t cs_rows = 0, int64_t cs_cols = 0,
                   int cs_accumulate = 0);
 
-// Bytes of GEMM scratch (split-K partials) that gemm_f32_core requests for
-// this shape: 0 when it runs without a split.
-size_t gemm_scratch_bytes(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_t batches);
+// Bytes of GEMM scratch (split-K partials) that gemm_f32_core requests at most
+// for this shape: 0 when it runs without a split.
+size_t gemm_scratch_bytes(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                          int64_t batches);
 
 inline int check_hip(hipError_t e, const char* where) {
   if (e != hipSuccess) {

@@ -1,4 +1,4 @@
-// fp32 GEMM on CDNA4 matrix cores (v_mfma_f32_32x32x2f32), ColMajor operands.
+// fp32 GEMM on CDNA4 matrix cores, ColMajor operands.
 //
 //   C[M,N] = alpha * op(A)[M,K] * op(B)[K,N] + beta * C (+ bias[n]) (ReLU)
 //
@@ -6,13 +6,19 @@
 // (forward NN, weight-grad TN, input-grad NT; ref: matmul.cu:16-71,
 // matmul_grad_weight.cu:14-69, matmul_grad_input.cu:14-68) and the batched
 // products of the recurrent and attention layers.  The reference computes one
-// output per thread with atomicAdd accumulation.  Here a block of
-// WGM x WGN wave64s owns a (WGM*WM*32) x (WGN*WN*32) output tile (up to
-// 256 x 128, each wave 128 x 64 as 4 x 2 MFMA blocks); K advances 16 at a
-// time through double-buffered, k-contiguous LDS tiles (mfma_kpack.hpp); no
-// atomics are used.  When the output tiles alone cannot fill the 256 CUs, K
-// is split across blocks into a stream-ordered workspace and the partials
-// are summed in a fixed order, so results are deterministic.
+// output per thread with atomicAdd accumulation.  Here a block of 8 wave64s
+// owns an output tile of up to 256 x 256 and forms it on the bf16 matrix
+// cores from operands split into three bf16 terms (mfma_split.hpp), with the
+// error of an fp32 sum; skinny products use fp32 MFMA tiles
+// (mfma_kpack.hpp), tiny ones plain FMAs; no atomics are used.  When the
+// output tiles alone cannot fill the 256 CUs, K is split across blocks into
+// a stream-ordered workspace and the partials are summed in a fixed order,
+// so results are deterministic.
+//
+// Measured on MI355X, fp32 MFMA tiles before -> split operands: 4096^3 980 ->
+// 625-640 us (219 TFLOP/s; the bf16 pipe alone would take 453 us at the
+// 1.82 PFLOP/s that the card's power limit leaves it), 8192 x 512 x 2048 144
+// -> 95 us, 8192 x 2048 x 512 160 -> 112 us, 32 x (256 x 512 x 256) 25 -> 21 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -23,30 +29,37 @@
 #include "colsum.hpp"
 #include "common.hpp"
 #include "mfma_kpack.hpp"
+#include "mfma_split.hpp"
 
 namespace cnhip {
 namespace {
 
 using kp::f32x16;
 using kp::f32x4;
+using sp::f32x4u;
 
-// Tile shapes (measured on MI355X: the 8-wave blocks keep two waves per SIMD
-// with 64x64 wave tiles and beat 4-wave blocks with larger wave tiles).
-using CfgXL = kp::Cfg<4, 2, 2, 2>;  // 256 x 128, 8 waves of 64x64
-using CfgXN = kp::Cfg<2, 4, 2, 2>;  // 128 x 256, 8 waves of 64x64
-using CfgXX = kp::Cfg<4, 4, 2, 2>;  // 256 x 256, 16 waves of 64x64 (one block per CU)
-using CfgM = kp::Cfg<4, 2, 1, 2>;   // 128 x 128, 8 waves of 32x64
-using CfgSN = kp::Cfg<4, 1, 1, 1>;  // 128 x 32 : N <= 32
-using CfgSM = kp::Cfg<1, 4, 1, 1>;  // 32 x 128 : M <= 32
-using CfgS = kp::Cfg<2, 2, 1, 1>;   // 64 x 64  : small problems
+// Tile shapes.  The products of large and medium shape run on the bf16 matrix
+// cores with their operands split in three (mfma_split.hpp), 8 waves a block;
+// the fp32 MFMA keeps the skinny ones, and operands whose rows lie so far
+// apart that 32-bit offsets do not span a tile.
+using CfgXX = kp::Cfg<2, 4, 4, 2>;           // 256 x 256, waves of 128x64, k whole
+using CfgM = kp::Cfg<2, 2, 2, 2, 16, 2>;     // 128 x 128, 2 k groups of 4 waves of 64x64
+using CfgN = kp::Cfg<2, 2, 2, 1, 16, 2>;     // 128 x 64, 2 k groups of 4 waves of 64x32
+using CfgQ = kp::Cfg<2, 2, 1, 1, 16, 2>;     // 64 x 64, 2 k groups of 4 waves of 32x32
+using CfgSN = kp::Cfg<4, 1, 1, 1>;           // 128 x 32 : N <= 32, fp32 MFMA
+using CfgSM = kp::Cfg<1, 4, 1, 1>;           // 32 x 128 : M <= 32, fp32 MFMA
+using CfgS = kp::Cfg<2, 2, 1, 1>;            // 64 x 64, fp32 MFMA: any leading dimension
+
+template <class C>
+constexpr bool split_cfg() { return C::NT == 512; }
 
 // Split-K granularity: a multiple of every tile shape's BK.
 constexpr int64_t KQ = 32;
 
-// Blocks of 512 threads run one per CU (their 64x64 wave tiles need ~150
-// VGPRs); 256-thread blocks are sized for two.
+// Waves per SIMD to leave registers for: the split shapes run one 8-wave
+// block per CU, the smallest of them two; the 4-wave fp32 shapes two.
 template <class C>
-constexpr int min_blocks() { return C::NT >= 512 ? 4 : 2; }
+constexpr int min_waves() { return split_cfg<C>() && C::BM * C::BN <= 64 * 64 ? 4 : 2; }
 
 struct GemmArgs {
   int64_t M, N, K;
@@ -64,10 +77,11 @@ struct GemmArgs {
   int64_t ld_aux;
   int vec_ok;            // every ld and stride % 4 == 0 and A, B 16-byte aligned
   int c_vec_ok;          // ldc, stride_c % 4 == 0 and C 16-byte aligned
-  int aux_vec_ok;        // ld_aux % 4 == 0 and aux_in 16-byte aligned
+  int aux_ok;            // aux_in given and one batch entry
   int64_t k_per_split;   // multiple of KQ (hence of every tile's BK)
   float* partial;        // split-K workspace [batch][splits][M*N]; null = direct
   int splits;
+  int park;              // 256 x 256 tile: C may hold a half sum before the result (no split, C not read)
   float* colsum;         // small kernels only: colsum[n] (+)= sum_k op(B)(k, n), or null
   int colsum_acc;        // 1: add to colsum, 0: overwrite
 };
@@ -166,9 +180,25 @@ __device__ __forceinline__ void gemm_mainloop(const GemmArgs& g, const float* __
   kp::pipeline<C>(ntiles, lds, s, acc);
 }
 
-// Epilogue of an interior tile (every row and column in range, C float4-
-// aligned, beta == 0, no split-K).  AUX: the fused epilogue reads aux_in
-// (DRELU, DGELU, ADD; aux_in float4-aligned), else it is NONE or RELU.
+// Accumulator block b (row-major over WM x WN) by a wave-uniform index.
+template <class C>
+__device__ __forceinline__ f32x16 acc_block(const f32x16 (&acc)[C::WM][C::WN], int b) {
+  f32x16 x = acc[0][0];
+  // value by value: a conditional copy of a whole block is turned into a load
+  // through a selected address, which puts the accumulators into memory
+#pragma unroll
+  for (int k = 1; k < C::WM * C::WN; ++k)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float y = acc[k / C::WN][k % C::WN][e];
+      x[e] = b == k ? y : x[e];
+    }
+  return x;
+}
+
+// Epilogue of an interior tile (every row and column in range, beta == 0, no
+// split-K).  AUX: the fused epilogue reads aux_in (DRELU, DGELU, ADD), else
+// it is NONE or RELU.  Its float4s need no 16-byte alignment (f32x4u).
 // The pointers are __restrict__ so loads may be scheduled ahead of stores
 // to C: the bias of every column the thread owns is loaded first, and per
 // 32 x 32 accumulator block the four aux float4s are loaded before the
@@ -189,46 +219,58 @@ __device__ __forceinline__ void epilogue_interior(const GemmArgs& g, float* __re
   constexpr int NB = C::WM * C::WN;
   auto col = [&](int b) { return n0 + wn * (C::WN * 32) + (b % C::WN) * 32 + (lane & 31); };
   auto row = [&](int b, int q) { return m0 + wm * (C::WM * 32) + (b / C::WN) * 32 + 8 * q + 4 * (lane >> 5); };
-  float bv[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) bv[b] = bias ? bias[col(b)] : 0.f;
-  f32x4 cur[4], nxt[4];
   if constexpr (AUX) {
+    // A real loop (unrolled, eight blocks of the GELU derivative are 20 K
+    // instructions): the block's accumulators are picked by a uniform branch.
+    f32x4 cur[4], nxt[4];
+    float bc = bias ? bias[col(0)] : 0.f, bn = 0.f;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) cur[q] = *reinterpret_cast<const f32x4*>(aux + row(0, q) + g.ld_aux * col(0));
-  }
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    if constexpr (AUX) {
+    for (int q = 0; q < 4; ++q) cur[q] = *reinterpret_cast<const f32x4u*>(aux + row(0, q) + g.ld_aux * col(0));
+#pragma unroll 1
+    for (int b = 0; b < NB; ++b) {
       if (b + 1 < NB) {
+        if (bias) bn = bias[col(b + 1)];
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          nxt[q] = *reinterpret_cast<const f32x4*>(aux + row(b + 1, q) + g.ld_aux * col(b + 1));
+          nxt[q] = *reinterpret_cast<const f32x4u*>(aux + row(b + 1, q) + g.ld_aux * col(b + 1));
       }
-    }
-    const int64_t n = col(b);
+      const f32x16 x = acc_block<C>(acc, b);
+      const int64_t n = col(b);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      f32x4 o;
+      for (int q = 0; q < 4; ++q) {
+        f32x4 o;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float v = g.alpha * acc[b / C::WN][b % C::WN][4 * q + e];
-        if (bias) v += bv[b];
-        if constexpr (AUX) {
+        for (int e = 0; e < 4; ++e) {
+          float v = g.alpha * x[4 * q + e];
+          if (bias) v += bc;
           const float a = cur[q][e];
           o[e] = g.epilogue == EPI_DRELU   ? v * relu_mask(a)
                  : g.epilogue == EPI_DGELU ? v * gelu_grad_f(a)
                                            : v + a;
-        } else {
+        }
+        *reinterpret_cast<f32x4u*>(Cp + row(b, q) + g.ldc * n) = o;
+      }
+      bc = bn;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) cur[q] = nxt[q];
+    }
+  } else {
+    float bv[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) bv[b] = bias ? bias[col(b)] : 0.f;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int64_t n = col(b);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float v = g.alpha * acc[b / C::WN][b % C::WN][4 * q + e];
+          if (bias) v += bv[b];
           o[e] = g.epilogue == CNHIP_EPI_RELU ? relu_f(v) : v;
         }
-      }
-      *reinterpret_cast<f32x4*>(Cp + row(b, q) + g.ldc * n) = o;
-    }
-    if constexpr (AUX) {
-      if (b + 1 < NB) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) cur[q] = nxt[q];
+        *reinterpret_cast<f32x4u*>(Cp + row(b, q) + g.ldc * n) = o;
       }
     }
   }
@@ -236,7 +278,8 @@ __device__ __forceinline__ void epilogue_interior(const GemmArgs& g, float* __re
 
 template <bool TA, bool TB, class C>
 constexpr int gemm_lds_floats() {
-  return 2 * kp::stage_floats<GemmStage<true, TA, TB, C>>();
+  if constexpr (split_cfg<C>()) return sp::Tile<TA, TB, C>::LDS / 4;
+  else return 2 * kp::stage_floats<GemmStage<true, TA, TB, C>>();
 }
 
 // One block of a GEMM launch: tile block `bx` (grid x), batch entry `batch`
@@ -255,17 +298,26 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& g, float* lds, int bx
   const int64_t k_begin = (int64_t)split * g.k_per_split;
   const int64_t k_end = min(g.K, k_begin + g.k_per_split);
   const bool full_mn = (m0 + BM <= g.M) && (n0 + BN <= g.N);
-  const bool fast = g.vec_ok && full_mn && ((k_end - k_begin) % C::BK == 0);
 
   f32x16 acc[C::WM][C::WN];
   kp::zero_acc<C>(acc);
-  if (fast) gemm_mainloop<true, TA, TB, C>(g, A, B, m0, n0, k_begin, k_end, lds, acc);
-  else gemm_mainloop<false, TA, TB, C>(g, A, B, m0, n0, k_begin, k_end, lds, acc);
+  if constexpr (split_cfg<C>()) {
+    using T = sp::Tile<TA, TB, C>;
+    const sp::Park park{g.park ? g.C + batch * g.stride_c : nullptr, g.ldc, g.M, g.N, m0, n0};
+    const bool tiny =
+        T::run(A, g.lda, B, g.ldb, g.M, g.N, m0, n0, k_begin, k_end, reinterpret_cast<char*>(lds), park, split & 1, acc);
+    if (C::WGK > 1 && threadIdx.x >= C::NT / C::WGK) return;  // group 0 holds the sums
+    if (T::needs_fp32(acc, tiny)) T::fp32(A, g.lda, B, g.ldb, g.M, g.N, m0, n0, k_begin, k_end, acc);
+  } else {
+    const bool fast = g.vec_ok && full_mn && ((k_end - k_begin) % C::BK == 0);
+    if (fast) gemm_mainloop<true, TA, TB, C>(g, A, B, m0, n0, k_begin, k_end, lds, acc);
+    else gemm_mainloop<false, TA, TB, C>(g, A, B, m0, n0, k_begin, k_end, lds, acc);
+  }
 
   float* Cp = g.C + batch * g.stride_c;
-  if (full_mn && g.c_vec_ok && !g.partial && g.beta == 0.f) {
+  if (full_mn && !g.partial && g.beta == 0.f) {
     if constexpr (FUSED) {
-      if ((g.epilogue == EPI_DRELU || g.epilogue == EPI_DGELU || g.epilogue == EPI_ADD) && g.aux_vec_ok) {
+      if ((g.epilogue == EPI_DRELU || g.epilogue == EPI_DGELU || g.epilogue == EPI_ADD) && g.aux_ok) {
         epilogue_interior<C, true>(g, Cp, g.aux_in, g.bias, acc, m0, n0);
         return;
       }
@@ -275,13 +327,12 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& g, float* lds, int bx
     }
   }
   float* P = g.partial ? g.partial + (batch * g.splits + split) * g.M * g.N : nullptr;
-  const bool p_vec = (g.M & 3) == 0;
-  kp::for_each_acc_run<C>(acc, [&](int ml, int nl, const f32x4& v) {
+  auto put = [&](int ml, int nl, const f32x4& v) {
     const int64_t m = m0 + ml, n = n0 + nl;
     if (n >= g.N) return;
     if (P) {
-      if (p_vec && m + 3 < g.M) {
-        *reinterpret_cast<f32x4*>(P + m + g.M * n) = v;
+      if (m + 3 < g.M) {
+        *reinterpret_cast<f32x4u*>(P + m + g.M * n) = v;
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -289,21 +340,38 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& g, float* lds, int bx
       }
       return;
     }
-    if (g.c_vec_ok && m + 3 < g.M) {
+    if (m + 3 < g.M) {
       f32x4 o;
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = epilogue_value<FUSED>(g, Cp, v[e], m + e, n);
-      *reinterpret_cast<f32x4*>(Cp + m + g.ldc * n) = o;
+      *reinterpret_cast<f32x4u*>(Cp + m + g.ldc * n) = o;
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (m + e < g.M) Cp[(m + e) + g.ldc * n] = epilogue_value<FUSED>(g, Cp, v[e], m + e, n);
     }
-  });
+  };
+  if constexpr (FUSED) {
+    // a real loop over the accumulator blocks, as in epilogue_interior
+    const int lane = threadIdx.x & 63;
+    int wm, wn, wk;
+    kp::wave_pos<C>(wm, wn, wk);
+#pragma unroll 1
+    for (int b = 0; b < C::WM * C::WN; ++b) {
+      const f32x16 x = acc_block<C>(acc, b);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        put(wm * (C::WM * 32) + (b / C::WN) * 32 + 8 * q + 4 * (lane >> 5),
+            wn * (C::WN * 32) + (b % C::WN) * 32 + (lane & 31),
+            f32x4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]});
+    }
+  } else {
+    kp::for_each_acc_run<C>(acc, put);
+  }
 }
 
 template <bool TA, bool TB, class C, bool FUSED>
-__global__ void __launch_bounds__(C::NT, min_blocks<C>()) gemm_f32_kernel(GemmArgs g) {
+__global__ void __launch_bounds__(C::NT, min_waves<C>()) gemm_f32_kernel(GemmArgs g) {
   __shared__ __align__(16) float lds[gemm_lds_floats<TA, TB, C>()];
   gemm_block<TA, TB, C, FUSED>(g, lds, (int)blockIdx.x, (int64_t)blockIdx.y, (int)blockIdx.z);
 }
@@ -311,13 +379,9 @@ __global__ void __launch_bounds__(C::NT, min_blocks<C>()) gemm_f32_kernel(GemmAr
 // Two independent GEMMs in one launch, both on tile shape C: blocks
 // [0, n1) run the first's (tiles1 x batches1 x splits1) blocks, the rest the
 // second's, each block exactly as in its own launch (so each product is
-// bit-identical to a launch of its own with the same plan).  A GEMM whose
-// tiles fill only one of the two block slots per CU (256 tiles of 128 x 128)
-// leaves every CU's matrix pipe idle while its single block loads its first
-// k-tiles and stores its results; a second GEMM's blocks in the other slot
-// fill those gaps.
+// bit-identical to a launch of its own with the same plan).
 template <bool TA1, bool TB1, bool F1, bool TA2, bool TB2, bool F2, class C>
-__global__ void __launch_bounds__(C::NT, min_blocks<C>()) gemm_pair_kernel(GemmArgs g1, GemmArgs g2, int n1,
+__global__ void __launch_bounds__(C::NT, min_waves<C>()) gemm_pair_kernel(GemmArgs g1, GemmArgs g2, int n1,
                                                                            int tiles1, int batches1, int tiles2,
                                                                            int batches2) {
   constexpr int F = gemm_lds_floats<TA1, TB1, C>() > gemm_lds_floats<TA2, TB2, C>()
@@ -557,7 +621,7 @@ TimingRec* hbm_timing_slot(const char* kernel, double bytes) {
 
 namespace {
 
-enum class Shape { XX, XL, XN, M, SN, SM, S };
+enum class Shape { XX, M, N, Q, SN, SM, S };
 
 template <class Cfg>
 int64_t tiles_of(int64_t M, int64_t N) {
@@ -571,47 +635,71 @@ struct Plan {
   int64_t kps;
 };
 
-// Tile shape and split-K plan of one GEMM; splits <= max_splits.
-// Cost model of one launch: dispatch rounds times the K-tiles of one split,
-// plus the fixed-order reduce of split-K partials (read splits + 1 times M*N
-// floats at ~5 TB/s, and a launch).  Block slots per round: the 512-thread
-// shapes are compiled for 4 waves per SIMD, so 2 blocks share a CU (512
-// slots); the 256-thread 64 x 64 and skinny tiles fit 4 per CU (1024).  A
-// split count that leaves a nearly empty last round costs a whole extra
-// round, so it is avoided.  `eff` is the measured MFMA efficiency of the
-// tile relative to the 64 x 64-per-wave tiles (smaller per-wave tiles load
-// more LDS bytes per MFMA).  Splits keep >= 4 K-tiles of 32.  Returns the
-// estimated seconds and the best split count.
-double split_cost(Shape shape, int64_t tiles, int64_t M, int64_t N, int64_t K, int64_t batches,
-                  int max_splits, bool may_split, int& splits) {
-  int64_t bm = 0, bn = 0;
-  double eff = 1.0;
+// Split-K partials of the split-operand shapes stay within this (the fixed
+// workspace of the no-allocation entry points, which run the same plans).
+constexpr int64_t kMaxPartialBytes = (int64_t)32 << 20;
+
+// What a tile shape costs: block slots of the chip, seconds per 32 of k of
+// one round of those slots, and seconds a round spends outside its k loop
+// (first loads, stores).  Fitted to sweeps of every shape and split count
+// over 28 sizes (from 4096 x 64 x 64 to 4096^3, all orientations): the plan
+// is within 5% of the best of them but for 1001 x 785 x 515 (8%).
+struct ShapeCost {
+  int64_t slots;
+  double t_tile, t_round;
+};
+
+ShapeCost shape_cost(Shape shape) {
   switch (shape) {
-    case Shape::XX: bm = CfgXX::BM; bn = CfgXX::BN; break;
-    case Shape::XL: bm = CfgXL::BM; bn = CfgXL::BN; break;
-    case Shape::XN: bm = CfgXN::BM; bn = CfgXN::BN; break;
-    case Shape::M: bm = CfgM::BM; bn = CfgM::BN; eff = 0.95; break;
-    case Shape::SN: bm = CfgSN::BM; bn = CfgSN::BN; eff = 0.8; break;
-    case Shape::SM: bm = CfgSM::BM; bn = CfgSM::BN; eff = 0.8; break;
-    case Shape::S: bm = CfgS::BM; bn = CfgS::BN; eff = 0.8; break;
+    case Shape::XX: return {256, 4.5e-6, 10e-6};
+    case Shape::M: return {256, 1.42e-6, 6e-6};
+    case Shape::N: return {256, 1.05e-6, 5e-6};
+    case Shape::Q: return {512, 1.34e-6, 4e-6};
+    case Shape::SN: return {1024, 2.0 * CfgSN::BM * CfgSN::BN * KQ / (157.3e12 / 256) * 4 / 0.8, 0};
+    case Shape::SM: return {1024, 2.0 * CfgSM::BM * CfgSM::BN * KQ / (157.3e12 / 256) * 4 / 0.8, 0};
+    case Shape::S: return {1024, 2.0 * CfgS::BM * CfgS::BN * KQ / (157.3e12 / 256) * 4 / 0.8, 0};
   }
-  const bool big = shape == Shape::XX || shape == Shape::XL || shape == Shape::XN || shape == Shape::M;
-  const int64_t per_cu = big ? 2 : 4;
-  const int64_t slots = 256 * per_cu;
-  // seconds per K-tile of 32 of one block, sharing its CU with per_cu - 1 others
-  const double t_tile = 2.0 * bm * bn * KQ / (157.3e12 / 256) * (double)per_cu / eff;
-  const int64_t blocks = tiles * batches;
+  return {1024, 1e-6, 0};
+}
+
+int64_t shape_tiles(Shape shape, int64_t M, int64_t N) {
+  switch (shape) {
+    case Shape::XX: return tiles_of<CfgXX>(M, N);
+    case Shape::M: return tiles_of<CfgM>(M, N);
+    case Shape::N: return tiles_of<CfgN>(M, N);
+    case Shape::Q: return tiles_of<CfgQ>(M, N);
+    case Shape::SN: return tiles_of<CfgSN>(M, N);
+    case Shape::SM: return tiles_of<CfgSM>(M, N);
+    case Shape::S: return tiles_of<CfgS>(M, N);
+  }
+  return 0;
+}
+
+// Cost of one launch: dispatch rounds times the k-tiles of one split, plus
+// the fixed-order reduce of split-K partials (read splits + 1 times M*N
+// floats, and a launch), over split counts min_s, 2 min_s, .. (INFINITY when
+// there is none).  A split count that leaves a nearly empty last round
+// costs a whole extra round, so it is avoided.  Splits keep >= 2 k-tiles of
+// 32 (4 for the fp32 shapes).  Returns the estimated seconds and the best
+// split count.
+double split_cost(Shape shape, int64_t M, int64_t N, int64_t K, int64_t batches, int max_splits, int& splits,
+                  int64_t min_s = 1) {
+  const ShapeCost c = shape_cost(shape);
+  const int64_t blocks = shape_tiles(shape, M, N) * batches;
+  const bool fp32 = shape == Shape::SN || shape == Shape::SM || shape == Shape::S;
   int64_t max_s = 1;
-  if (may_split && blocks < slots && K >= 8 * KQ)
-    max_s = std::max<int64_t>(1, std::min<int64_t>(K / (4 * KQ), max_splits));
+  if (blocks < c.slots && K >= 8 * KQ)
+    max_s = std::max<int64_t>(1, std::min<int64_t>(K / ((fp32 ? 4 : 2) * KQ), max_splits));
+  if (!fp32) max_s = std::max<int64_t>(1, std::min<int64_t>(max_s, kMaxPartialBytes / (M * N * batches * 4)));
+  if (max_s < min_s) return INFINITY;
   double best = 0.0;
   splits = 1;
-  for (int64_t s = 1; s <= max_s; ++s) {
+  for (int64_t s = min_s; s <= max_s; s += min_s) {
     const int64_t kt = ((K + s - 1) / s + KQ - 1) / KQ;
-    const int64_t rounds = (blocks * s + slots - 1) / slots;
-    double cost = (double)rounds * (double)kt * t_tile;
+    const int64_t rounds = (blocks * s + c.slots - 1) / c.slots;
+    double cost = (double)rounds * ((double)kt * c.t_tile + c.t_round);
     if (s > 1) cost += (double)(s + 1) * M * N * batches * 4.0 / 5e12 + 3e-6;
-    if (s == 1 || cost < best) {
+    if (s == min_s || cost < best) {
       best = cost;
       splits = (int)s;
     }
@@ -619,73 +707,43 @@ double split_cost(Shape shape, int64_t tiles, int64_t M, int64_t N, int64_t K, i
   return best;
 }
 
-Plan plan_gemm(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_t batches,
-               int max_splits) {
-  // Skinny shapes take the 32-wide tiles (no MFMA work on padding), split by
-  // the cost model above.  Otherwise, in order (rules fitted to measured
-  // tile x split sweeps on MI355X, where the 512-thread tiles run 2 blocks
-  // per CU and split-K costs more than its reduce traffic alone):
-  //   128 x 256 (256 x 128 when only A is k-contiguous) if >= 512 blocks,
-  //   256 x 256 instead when that gives whole rounds of 256 blocks, K >= 1024;
-  //   128 x 128 if >= 256 blocks;  64 x 64 if >= 512 blocks;
-  //   else split K: 128 x 128 toward 512 blocks (<= 16 splits) if that
-  //   reaches 256 blocks, otherwise 64 x 64 toward 512 blocks.
-  Shape shape;
+// Below this contraction the half sum that a 256 x 256 tile parks in C costs
+// more (45 us for 256 tiles) than the tile gains over 128 x 128: measured
+// 4096 x 4096 x 1024 at 201 us against 196, x 4096 at 638 against 716.
+constexpr int64_t kParkMinK = 1536;
+
+// A 256 x 256 tile without a half sum in C takes an even number of splits.
+// can_park: C is neither read (beta) nor the memory of the side tensor.
+Plan plan_gemm(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t batches,
+               bool can_park, int max_splits) {
+  // Skinny shapes take the 32-wide fp32 tiles (no MFMA work on padding), the
+  // rest the split shape and split count of the lowest cost.
+  Shape shape = Shape::S;
   int splits = 1;
   if (N <= 32 || M <= 32) {
     shape = N <= 32 ? Shape::SN : Shape::SM;
-    split_cost(shape, shape == Shape::SN ? tiles_of<CfgSN>(M, N) : tiles_of<CfgSM>(M, N), M, N, K,
-               batches, max_splits, true, splits);
+    split_cost(shape, M, N, K, batches, max_splits, splits);
+  } else if (K < sp::KT || !sp::offsets_fit(lda, trans_a != 0, CfgXX::BM) || !sp::offsets_fit(ldb, trans_b == 0, CfgXX::BN)) {
+    split_cost(shape, M, N, K, batches, max_splits, splits);
   } else {
-    const bool a_kc = trans_a != 0, b_kc = trans_b == 0;
-    const Shape big = (a_kc && !b_kc) ? Shape::XL : Shape::XN;
-    const int64_t tb = (big == Shape::XL ? tiles_of<CfgXL>(M, N) : tiles_of<CfgXN>(M, N)) * batches;
-    const int64_t tm = tiles_of<CfgM>(M, N) * batches;
-    const int64_t ts = tiles_of<CfgS>(M, N) * batches;
-    const int64_t max_s = K >= 8 * KQ ? std::max<int64_t>(1, std::min<int64_t>(K / (4 * KQ), max_splits)) : 1;
-    if (tb >= 512) {
-      // whole rounds of 256 x 256 tiles (one 16-wave block per CU) for a
-      // long contraction: each staged k-tile feeds 16 waves instead of 8
-      // (config 2's 4096^3 GEMMs 0.6-1.7% faster than 128 x 256)
-      const int64_t tx = tiles_of<CfgXX>(M, N) * batches;
-      shape = K >= 1024 && tx % 256 == 0 ? Shape::XX : big;
-    } else if (tm >= 256) {
-      shape = Shape::M;
-    } else if (ts >= 512) {
-      shape = Shape::S;
-    } else {
-      // too few tiles to fill the chip: split K.  The 128 x 128 tile's split
-      // count (<= 16) is the one with the lowest dispatch-round cost: a count
-      // that leaves some CUs a block more than the others costs that block's
-      // whole duration (11 splits of 48 tiles, 528 blocks, ran at 82 TFLOP/s
-      // where 10 splits, 480 blocks, run at 92)
-      int sm = 1;
-      split_cost(Shape::M, tm / batches, M, N, K, batches, (int)std::min<int64_t>(16, max_s), true, sm);
-      if (tm * sm >= 256) {
-        shape = Shape::M;
-        splits = sm;
-      } else {
-        shape = Shape::S;
-        splits = (int)std::min<int64_t>((512 + ts - 1) / ts, max_s);
+    double best = 0.0;
+    for (Shape c : {Shape::XX, Shape::M, Shape::N, Shape::Q}) {
+      int sc = 1;
+      const bool whole = c != Shape::XX || (can_park && K >= kParkMinK);
+      const double cost = split_cost(c, M, N, K, batches, std::min(max_splits, 16), sc, whole ? 1 : 2);
+      if (c == Shape::XX || cost < best) {
+        best = cost;
+        shape = c;
+        splits = sc;
       }
     }
-  }
-  int64_t tiles = 0;
-  switch (shape) {
-    case Shape::XX: tiles = tiles_of<CfgXX>(M, N); break;
-    case Shape::XL: tiles = tiles_of<CfgXL>(M, N); break;
-    case Shape::XN: tiles = tiles_of<CfgXN>(M, N); break;
-    case Shape::M: tiles = tiles_of<CfgM>(M, N); break;
-    case Shape::SN: tiles = tiles_of<CfgSN>(M, N); break;
-    case Shape::SM: tiles = tiles_of<CfgSM>(M, N); break;
-    case Shape::S: tiles = tiles_of<CfgS>(M, N); break;
   }
   int64_t kps = (K + splits - 1) / splits;
   kps = ((kps + KQ - 1) / KQ) * KQ;
   if (kps == 0) kps = KQ;
   splits = K > 0 ? (int)((K + kps - 1) / kps) : 1;
 
-  return Plan{shape, tiles, splits, kps};
+  return Plan{shape, shape_tiles(shape, M, N), splits, kps};
 }
 
 // Launches the planned kernel, bracketed by the per-launch timing events.
@@ -696,9 +754,9 @@ int launch_plan(Shape shape, int trans_a, int trans_b, const GemmArgs& g, int64_
   if (rec) (void)hipEventRecord(rec->start, st);
   switch (shape) {
     case Shape::XX: launch_t<CfgXX>(trans_a, trans_b, g, batches, st); break;
-    case Shape::XL: launch_t<CfgXL>(trans_a, trans_b, g, batches, st); break;
-    case Shape::XN: launch_t<CfgXN>(trans_a, trans_b, g, batches, st); break;
     case Shape::M: launch_t<CfgM>(trans_a, trans_b, g, batches, st); break;
+    case Shape::N: launch_t<CfgN>(trans_a, trans_b, g, batches, st); break;
+    case Shape::Q: launch_t<CfgQ>(trans_a, trans_b, g, batches, st); break;
     case Shape::SN: launch_t<CfgSN>(trans_a, trans_b, g, batches, st); break;
     case Shape::SM: launch_t<CfgSM>(trans_a, trans_b, g, batches, st); break;
     case Shape::S: launch_t<CfgS>(trans_a, trans_b, g, batches, st); break;
@@ -790,10 +848,12 @@ static size_t split_bytes(const Plan& plan, int64_t M, int64_t N, int64_t batche
   return plan.splits > 1 ? (size_t)batches * (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
-size_t gemm_scratch_bytes(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_t batches) {
+size_t gemm_scratch_bytes(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                          int64_t batches) {
   if (M <= 0 || N <= 0 || K < 0 || batches <= 0) return 0;
   if (gemm_is_small(M, N, K, batches, trans_a, trans_b)) return 0;
-  return split_bytes(plan_gemm(trans_a, trans_b, M, N, K, batches, 64), M, N, batches);
+  return std::max(split_bytes(plan_gemm(trans_a, trans_b, M, N, K, lda, ldb, batches, true, 64), M, N, batches),
+                  split_bytes(plan_gemm(trans_a, trans_b, M, N, K, lda, ldb, batches, false, 64), M, N, batches));
 }
 
 
@@ -813,6 +873,17 @@ static int check_spec(const GemmSpec& s, const char* who) {
   return CNHIP_OK;
 }
 
+// Whether C may hold an intermediate half sum: it is not read (beta) and no
+// element of the side tensor lies in it (a residual added in place).
+static bool can_park(const GemmSpec& s) {
+  if (s.beta != 0.f) return false;
+  auto apart = [&](const float* aux) {
+    const float* c_end = s.C + s.stride_c * (s.batches - 1) + s.ldc * (s.N - 1) + s.M;
+    return !aux || aux >= c_end || aux + s.ld_aux * (s.N - 1) + s.M <= s.C;
+  };
+  return apart(s.aux_in) && apart(s.aux_out);
+}
+
 static GemmArgs args_of(const GemmSpec& s, const Plan& plan) {
   GemmArgs g;
   g.M = s.M; g.N = s.N; g.K = s.K;
@@ -824,10 +895,11 @@ static GemmArgs args_of(const GemmSpec& s, const Plan& plan) {
   g.vec_ok = (s.lda % 4 == 0) && (s.ldb % 4 == 0) && (s.stride_a % 4 == 0) && (s.stride_b % 4 == 0) &&
              aligned16(s.A) && aligned16(s.B);
   g.c_vec_ok = (s.ldc % 4 == 0) && (s.stride_c % 4 == 0) && aligned16(s.C);
-  g.aux_vec_ok = (s.ld_aux % 4 == 0) && s.aux_in && aligned16(s.aux_in) && s.batches == 1;
+  g.aux_ok = s.aux_in && s.batches == 1;
   g.partial = nullptr;
   g.k_per_split = plan.kps;
   g.splits = plan.splits;
+  g.park = plan.shape == Shape::XX && plan.splits == 1;
   g.colsum = nullptr;
   g.colsum_acc = 0;
   return g;
@@ -877,7 +949,7 @@ static int gemm_spec(const GemmSpec& s, hipStream_t st, const char* who, const C
     return sums();
   }
 
-  const Plan plan = plan_gemm(s.trans_a, s.trans_b, s.M, s.N, s.K, s.batches, 64);
+  const Plan plan = plan_gemm(s.trans_a, s.trans_b, s.M, s.N, s.K, s.lda, s.ldb, s.batches, can_park(s), 64);
   CNHIP_REQUIRE(plan.tiles < ((int64_t)1 << 30), "%s: GEMM too large", who);
   GemmArgs g = args_of(s, plan);
   if (plan.splits > 1) {
@@ -905,44 +977,25 @@ int gemm_f32_core(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, flo
 // epilogue) of the first, then of the second.
 #define CNHIP_PAIR_CODE(a1, b1, f1, a2, b2, f2) ((a1) << 5 | (b1) << 4 | (f1) << 3 | (a2) << 2 | (b2) << 1 | (f2))
 
-// x (an input gradient, NT) and y (a TN weight gradient) that both plan to
-// the 256 x 256 tile without split-K, in one launch of tiles_x + tiles_y
-// blocks: each CU runs one such block at a time, so the launch is the two
-// GEMMs' rounds back to back, and a CU whose block of x has finished starts
-// a block of y while the others still store x's tiles (as separate launches,
-// every CU waits for the last tile of x and for the end-of-kernel writeback).
-// Each block computes exactly as in its own launch.
-static int pair_xx(const GemmSpec& x, const GemmSpec& y, const Plan& px, const Plan& py, bool fx, hipStream_t st,
-            const char* who, const ColsumJob* cs) {
-  using C = CfgXX;
-  const void* kern = nullptr;
-  if (x.trans_a == 0 && x.trans_b == 1 && y.trans_a == 1 && y.trans_b == 0)
-    kern = fx ? (const void*)&gemm_pair_kernel<false, true, true, true, false, false, C>
-              : (const void*)&gemm_pair_kernel<false, true, false, true, false, false, C>;
-  if (!kern) {
-    CNHIP_TRY(gemm_spec(x, st, who));
-    return gemm_spec(y, st, who, cs);
+// The pair kernel for two GEMMs on tile shape C, or null when no instance
+// serves their orientations.  Pairs served: x an input gradient (NT,
+// optionally with a fused epilogue) or a TN product, y a TN weight gradient
+// or an NN product.
+template <class C>
+static const void* pair_kernel(int code) {
+  switch (code) {
+    case CNHIP_PAIR_CODE(0, 1, 1, 1, 0, 0): return (const void*)&gemm_pair_kernel<false, true, true, true, false, false, C>;
+    case CNHIP_PAIR_CODE(0, 1, 0, 1, 0, 0): return (const void*)&gemm_pair_kernel<false, true, false, true, false, false, C>;
+    case CNHIP_PAIR_CODE(1, 0, 0, 0, 0, 0): return (const void*)&gemm_pair_kernel<true, false, false, false, false, false, C>;
+    default: return nullptr;
   }
-  GemmArgs gx = args_of(x, px), gy = args_of(y, py);
-  const int64_t nx = px.tiles * x.batches, ny = py.tiles * y.batches;
-  TimingRec* rec = timing_slot(2.0 * (double)x.M * (double)x.N * (double)x.K * (double)x.batches +
-                               2.0 * (double)y.M * (double)y.N * (double)y.K * (double)y.batches);
-  if (rec) (void)hipEventRecord(rec->start, st);
-  const int n1 = (int)nx, t1 = (int)px.tiles, b1 = (int)x.batches, t2 = (int)py.tiles, b2 = (int)y.batches;
-  void* kargs[] = {&gx, &gy, const_cast<int*>(&n1), const_cast<int*>(&t1), const_cast<int*>(&b1),
-                   const_cast<int*>(&t2), const_cast<int*>(&b2)};
-  int status = check_hip(hipLaunchKernel(kern, dim3((unsigned)(nx + ny)), dim3(C::NT), kargs, 0, st), who);
-  if (status == CNHIP_OK) status = check_launch(who);
-  if (rec) (void)hipEventRecord(rec->stop, st);
-  if (status != CNHIP_OK) return status;
-  return cs ? column_sum(cs->in, cs->out, cs->rows, cs->cols, cs->accumulate, st, who) : CNHIP_OK;
 }
 
-// x and y in one launch when both take the 128 x 128 tile, x does not split
-// K, and together they fit the chip's 512 block slots at once (y's split
-// count is lowered to fit, never raised); otherwise one after the other.
-// Pairs served: x an input gradient (NT, optionally with a fused epilogue)
-// or a TN product, y a TN weight gradient or an NN product.
+// x and y in one launch when both take the same tile shape and x does not
+// split K; otherwise one after the other.  A CU whose block of x has finished
+// starts a block of y while the others still store x's tiles (as separate
+// launches, every CU waits for the last tile of x and for the end-of-kernel
+// writeback).  Each block computes exactly as in its own launch.
 int gemm_f32_pair(const GemmSpec& x, const GemmSpec& y, hipStream_t st, const char* who, const float* cs_in,
                   float* cs_out, int64_t cs_rows, int64_t cs_cols, int cs_accumulate) {
   CNHIP_TRY(check_spec(x, who));
@@ -961,46 +1014,29 @@ int gemm_f32_pair(const GemmSpec& x, const GemmSpec& y, hipStream_t st, const ch
            !gemm_is_small(s.M, s.N, s.K, s.batches, s.trans_a, s.trans_b);
   };
   if (!big(x) || !big(y)) return apart();
-  const Plan px = plan_gemm(x.trans_a, x.trans_b, x.M, x.N, x.K, x.batches, 64);
-  Plan py = plan_gemm(y.trans_a, y.trans_b, y.M, y.N, y.K, y.batches, 64);
+  const Plan px = plan_gemm(x.trans_a, x.trans_b, x.M, x.N, x.K, x.lda, x.ldb, x.batches, can_park(x), 64);
+  const Plan py = plan_gemm(y.trans_a, y.trans_b, y.M, y.N, y.K, y.lda, y.ldb, y.batches, can_park(y), 64);
+  if (px.shape != py.shape || px.splits != 1) return apart();
   const bool fx = !x.trans_a && x.epilogue >= EPI_GELU;
-  if (px.shape == Shape::XX && py.shape == Shape::XX && px.splits == 1 && py.splits == 1)
-    return pair_xx(x, y, px, py, fx, st, who, sums ? &cs : nullptr);
-  if (px.shape != Shape::M || py.shape != Shape::M || px.splits != 1) return apart();
-  constexpr int64_t kSlots = 512;  // 2 blocks of 512 threads per CU, 256 CUs
-  const int64_t nx = px.tiles * x.batches, ty = py.tiles * y.batches;
-  if (nx + ty > kSlots) return apart();
-  if (nx + ty * py.splits > kSlots) {
-    const int fit = (int)((kSlots - nx) / ty);
-    int64_t kps = (y.K + fit - 1) / fit;
-    kps = ((kps + KQ - 1) / KQ) * KQ;
-    py.kps = kps;
-    py.splits = (int)((y.K + kps - 1) / kps);
-  }
-  const bool fy = !y.trans_a && y.epilogue >= EPI_GELU;
-  const int code = CNHIP_PAIR_CODE(x.trans_a, x.trans_b, fx ? 1 : 0, y.trans_a, y.trans_b, fy && py.splits == 1 ? 1 : 0);
-  using C = CfgM;
-  const void* kern = nullptr;
-  switch (code) {
-    case CNHIP_PAIR_CODE(0, 1, 1, 1, 0, 0): kern = (const void*)&gemm_pair_kernel<false, true, true, true, false, false, C>; break;
-    case CNHIP_PAIR_CODE(0, 1, 0, 1, 0, 0): kern = (const void*)&gemm_pair_kernel<false, true, false, true, false, false, C>; break;
-    case CNHIP_PAIR_CODE(1, 0, 0, 0, 0, 0): kern = (const void*)&gemm_pair_kernel<true, false, false, false, false, false, C>; break;
-    default: return apart();
-  }
+  const bool fy = !y.trans_a && y.epilogue >= EPI_GELU && py.splits == 1;
+  const int code = CNHIP_PAIR_CODE(x.trans_a, x.trans_b, fx ? 1 : 0, y.trans_a, y.trans_b, fy ? 1 : 0);
+  const void* kern = px.shape == Shape::XX ? pair_kernel<CfgXX>(code) : px.shape == Shape::M ? pair_kernel<CfgM>(code)
+                                                                                            : nullptr;
+  const int64_t nx = px.tiles * x.batches, ny = py.tiles * y.batches * py.splits;
+  if (!kern || nx + ny >= ((int64_t)1 << 31)) return apart();
   GemmArgs gx = args_of(x, px), gy = args_of(y, py);
   if (py.splits > 1) {
     void* ws = nullptr;
     CNHIP_TRY(scratch(st, kScratchGemm, split_bytes(py, y.M, y.N, y.batches), &ws, who));
     gy.partial = static_cast<float*>(ws);
   }
-  const int64_t ny = ty * py.splits;
   TimingRec* rec = timing_slot(2.0 * (double)x.M * (double)x.N * (double)x.K * (double)x.batches +
                                2.0 * (double)y.M * (double)y.N * (double)y.K * (double)y.batches);
   if (rec) (void)hipEventRecord(rec->start, st);
   const int n1 = (int)nx, t1 = (int)px.tiles, b1 = (int)x.batches, t2 = (int)py.tiles, b2 = (int)y.batches;
   void* kargs[] = {&gx, &gy, const_cast<int*>(&n1), const_cast<int*>(&t1), const_cast<int*>(&b1),
                    const_cast<int*>(&t2), const_cast<int*>(&b2)};
-  int status = check_hip(hipLaunchKernel(kern, dim3((unsigned)(nx + ny)), dim3(C::NT), kargs, 0, st), who);
+  int status = check_hip(hipLaunchKernel(kern, dim3((unsigned)(nx + ny)), dim3(512), kargs, 0, st), who);
   if (status == CNHIP_OK) status = check_launch(who);
   if (rec) (void)hipEventRecord(rec->stop, st);
   if (status != CNHIP_OK) return status;

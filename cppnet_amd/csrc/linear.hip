@@ -434,8 +434,8 @@ size_t linear_backward_act_scratch_bytes(const float* X, const float* W, const f
                                   act == CNHIP_ACT_RELU || act == CNHIP_ACT_GELU ? act_aux : nullptr);
   const bool one_pass =
       full || (run && act != CNHIP_ACT_NONE && skinny_serves(B, I, O, X, W, dY, grad_W, nullptr, nullptr));
-  size_t need = one_pass ? skinny_bytes(B, I, O) : trainable ? gemm_scratch_bytes(1, 0, I, O, B, 1) : 0;
-  if (dX && !full) need = std::max(need, gemm_scratch_bytes(0, 1, B, I, O, 1));
+  size_t need = one_pass ? skinny_bytes(B, I, O) : trainable ? gemm_scratch_bytes(1, 0, I, O, B, B, B, 1) : 0;
+  if (dX && !full) need = std::max(need, gemm_scratch_bytes(0, 1, B, I, O, B, I, 1));
   return need;
 }
 

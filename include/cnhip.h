@@ -101,7 +101,8 @@ int cnhip_graph_destroy(cnhip_graph_t graph);
  *   trans_a == 0: A(m,k) = A[m + lda*k];  trans_a == 1: A(m,k) = A[k + lda*m]
  *   trans_b == 0: B(k,n) = B[k + ldb*n];  trans_b == 1: B(k,n) = B[n + ldb*k]
  * beta == 0 never reads C.  bias may be NULL.  epilogue: 0 none, 1 ReLU
- * applied after bias.  fp32 in, fp32 MFMA (v_mfma_f32_32x32x2f32), fp32 out.
+ * applied after bias.  fp32 in, fp32 out, with the error of an fp32 sum
+ * (fp32 MFMA, or bf16 MFMA over operands split exactly into three terms).
  * ref: src/CppNet/kernels/gpu/matmul.cu:16-71 (NN), matmul_grad_input.cu:14-68
  * (NT), matmul_grad_weight.cu:14-69 (TN), add_bias.cu:13-22 (bias epilogue). */
 #define CNHIP_EPI_NONE 0

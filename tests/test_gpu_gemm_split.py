@@ -1,0 +1,106 @@
+"""The GEMM shapes that run on the bf16 matrix cores with operands split in
+three: tile edges, remainders of K, odd leading dimensions and unaligned
+operands, every orientation and tile shape, against float64; and what bf16
+terms cannot hold (infinities, NaN, values near the ends of the fp32 range),
+against IEEE fp32 semantics."""
+import numpy as np
+import pytest
+import torch
+
+from cppnet_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def operand(gen, trans, rows, k, pad, off):
+    """X(r, k), k-contiguous when trans, as a flat tensor at an element offset."""
+    ld = (k if trans else rows) + pad
+    flat = torch.randn(ld * (rows if trans else k) + off, generator=gen, device="cuda")
+    x = flat[off:]
+    m = x.view(rows, ld)[:, :k] if trans else x.view(k, ld)[:, :rows].T
+    return x, m, ld
+
+
+# (M, N, K, batch): 64 x 64, 128 x 64, 128 x 128 tiles with and without
+# split-K, then 256 x 256 tiles (whole, with edges, split over K)
+SHAPES = [(65, 63, 700, 1), (100, 515, 2000, 1), (257, 129, 33, 40), (1001, 515, 785, 1), (2000, 130, 70, 1),
+          (8192, 512, 512, 1), (515, 517, 8191, 1), (256, 250, 500, 32), (4096, 4096, 2048, 1), (4090, 4087, 2051, 1),
+          (1024, 4096, 4096, 1)]
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("M,N,K,batch", SHAPES)
+def test_gemm_split_matches_float64(gpu, ta, tb, M, N, K, batch):
+    gen = torch.Generator("cuda").manual_seed(M + 3 * N + 7 * K + ta + 2 * tb)
+    if batch > 1:
+        A = torch.randn(batch, *((M, K) if ta else (K, M)), generator=gen, device="cuda")
+        B = torch.randn(batch, *((K, N) if tb else (N, K)), generator=gen, device="cuda")
+        C = torch.empty(batch, N, M, device="cuda")
+        ops.gemm_batched(bool(ta), bool(tb), M, N, K, A, K if ta else M, M * K, B, N if tb else K, N * K, C, M, M * N,
+                         batch)
+        a = (A if ta else A.transpose(1, 2)).double().contiguous()
+        b = (B if tb else B.transpose(1, 2)).double().contiguous()
+        got, want = C.transpose(1, 2).double(), torch.bmm(a, b)
+        size = torch.bmm(a.square(), b.square())
+    else:
+        x, a, lda = operand(gen, ta, M, K, 1 if K < 2000 else 0, 1)
+        y, b, ldb = operand(gen, not tb, N, K, 3 if K < 2000 else 0, 3)
+        pad = torch.full(((M + 5) * N,), 7.0, device="cuda")
+        ops.gemm(bool(ta), bool(tb), M, N, K, x, lda, y, ldb, pad, M + 5)
+        C = pad.view(N, M + 5)
+        assert bool((C[:, M:] == 7.0).all()), "wrote past the rows of C"
+        a, b = a.double().contiguous(), b.T.double().contiguous()
+        got, want, size = C[:, :M].T.double(), a @ b, a.square() @ b.square()
+    # An fp32 sum of K zero-mean products: partial sums grow to sqrt(sum
+    # (ab)^2), each rounding adds 2^-24 of one, so the error is ~ 2^-24
+    # sqrt(K/2) sqrt(sum (ab)^2) rms; 8 of these covers 16 M outputs.
+    lim = 8 * 2.0 ** -24 * (K / 2) ** 0.5 * size.sqrt()
+    err = (got - want).abs()
+    assert bool((err <= lim).all()), f"worst error / bound {float((err / lim).max()):.3g}"
+    # and its mean keeps no drift: 6 standard errors of a mean of M N batch
+    # such errors
+    rms = float(want.square().mean().sqrt())
+    assert abs(float((got - want).mean())) <= (6 / (M * N * batch) ** 0.5 + 0.02) * 2.0 ** -24 * (K / 2) ** 0.5 * rms
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 80, 700), (1001, 515, 785), (4096, 4096, 2048)])
+def test_gemm_split_nonfinite_and_range_ends(gpu, M, N, K):
+    gen = torch.Generator("cuda").manual_seed(K)
+    A = torch.randn(K, M, generator=gen, device="cuda")  # A(m, k) at [k, m]
+    B = torch.randn(N, K, generator=gen, device="cuda")
+    A[3, 5] = float("inf")
+    A[4, 7] = float("nan")
+    A[9, 11] = 3.4e38       # its bf16 term is infinite
+    B[:, 9] = B[:, 9].clamp(-0.5, 0.5)
+    B[13, K - 1] = float("-inf")
+    A[:, 17] = A[:, 17] * 1e-36
+    A[:, 19] = A[:, 19] * 2.0 ** -128  # subnormal
+    C = torch.empty(N, M, device="cuda")
+    ops.gemm(False, False, M, N, K, A, M, B, K, C, M)
+    want = (B.double() @ A.double())
+    got = C.double()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf())
+    assert bool((got[want.isinf()] == want[want.isinf()]).all())
+    ok = want.isfinite()
+    size = (B.double().square() @ A.double().square()).sqrt()
+    # 2^-149: half of the smallest subnormal for each of K products
+    lim = 8 * 2.0 ** -24 * (K / 2) ** 0.5 * size + K * 2.0 ** -149
+    assert bool(((got - want).abs()[ok] <= lim[ok]).all()), float(((got - want).abs()[ok] / lim[ok]).max())
+
+
+def test_linear_residual_in_place(gpu):
+    """The skip branch added into its own buffer (Z is Y): a tile whose half
+    sums would wait in C must not clobber it."""
+    B, I, O = 4096, 2048, 4096
+    gen = torch.Generator("cuda").manual_seed(5)
+    X = torch.randn(I, B, generator=gen, device="cuda")
+    W = torch.randn(O, I, generator=gen, device="cuda") / I ** 0.5
+    b = torch.randn(O, generator=gen, device="cuda")
+    Z = torch.randn(O, B, generator=gen, device="cuda")
+    Y = torch.empty_like(Z)
+    ops.linear_forward_act(X, W, b, Y, Z, B, I, O, "residual")
+    want = W.double() @ X.double() + b.double()[:, None] + Z.double()
+    assert float((Y.double() - want).abs().max()) < 1e-4
+    ops.linear_forward_act(X, W, b, Z, Z, B, I, O, "residual")
+    assert float((Z.double() - want).abs().max()) < 1e-4
