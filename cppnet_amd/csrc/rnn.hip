@@ -1055,6 +1055,273 @@ __global__ void __launch_bounds__(LstmBwdCfg::NT) lstm_step_bwd_kernel(
   dc_buf[e] = dcn;
 }
 
+// ---------------------------------------------------------------- persistent GRU
+// The GRU recurrence in one launch per pass, on the LSTM's tiles, placement
+// and exchange (above), for any B and any H up to 512: a block owns 16
+// samples x 16 hidden units, rows and columns past B and H enter as zeros and
+// are never stored, and HP = 64, 128, 256 or 512 is the padded width of the
+// contraction (words of units past the last tile are not waited for).
+//
+// A GRU step needs two exchanges, because r * h_{t-1} (forward) and dr
+// (backward) of every unit follow from a first product over all units.  The
+// per-step launches this replaces ran two split-K GEMMs, their reduces and
+// two cell kernels per step and pass: 27 us a step and pass at B 128, H 512,
+// nearly all of it launches and first loads (1.1 us of MFMA work); bound by
+// the two hand-overs (about 3 us each), a step here takes 7 us forward and
+// 8 us backward.
+//
+// Every product's k-blocks of 16 are dealt to the 4 waves (fp32 MFMA
+// 16 x 16 x 4, lane (q, r) supplying k = 16 kb + 4 q + e), whose partial
+// tiles are added in a fixed order by the cell threads; each wave's weights
+// stay in registers (3 HP / 16 float4s).  A gathered [16 samples x HP] vector
+// is staged in LDS as [k/4][sample].
+struct GruPersistArgs {
+  float* gates;       // forward: x W_ih in, activations out; backward: read
+  const float* bias;  // forward
+  float* Y;           // forward: written; backward: read
+  float* rh;          // forward: r * h_{t-1}
+  const float* dY;    // backward
+  float* dG;          // backward: written
+  const float* W_hh;
+  u64* ex;            // areas of [2 slots][nst][NUT 16][16] words
+  int B, S, H, nst;
+  PersistSync sync;
+};
+
+// Thread tid's words of a gathered vector: units tid / 8 + 32 j, samples
+// 2 (tid % 8) and the next; those at or past `units` are zeros already.
+template <int N, int SLEEP>
+__device__ __forceinline__ void gru_gather_issue(__amdgpu_buffer_rsrc_t rs, unsigned soff, unsigned stamp, int units,
+                                                 u32x4 (&w)[N]) {
+  if constexpr (SLEEP > 0) __builtin_amdgcn_s_sleep(SLEEP);
+  asm volatile("buffer_inv sc0" ::: "memory");
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    if (((int)threadIdx.x >> 3) + 32 * j < units)
+      w[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, threadIdx.x * 16u, soff + j * 4096u, 2);
+    else
+      w[j] = u32x4{0u, stamp, 0u, stamp};
+  }
+}
+template <int N>
+__device__ __forceinline__ void gru_stage(f32x4* tile, const u32x4 (&w)[N]) {
+  float* f = reinterpret_cast<float*>(tile);
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int k = ((int)threadIdx.x >> 3) + 32 * j, s2 = 2 * ((int)threadIdx.x & 7);
+    f[((k >> 2) * kPt + s2) * 4 + (k & 3)] = __uint_as_float(w[j].x);
+    f[((k >> 2) * kPt + s2 + 1) * 4 + (k & 3)] = __uint_as_float(w[j].z);
+  }
+}
+// acc += tile[16 samples, k-blocks kb0 .. kb0 + N) times the wave's weights.
+template <int N>
+__device__ __forceinline__ void gru_product(const f32x4* tile, int kb0, const f32x4 (&wv)[N], f32x4& acc) {
+  const int lane = threadIdx.x & 63, q = lane >> 4, r = lane & 15;
+  f32x4 odd = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const f32x4 v = tile[(4 * (kb0 + k) + q) * kPt + r];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (k & 1) odd = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], wv[k][e], odd, 0, 0, 0);
+      else acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], wv[k][e], acc, 0, 0, 0);
+    }
+  }
+  acc += odd;
+}
+
+template <int HP>
+__global__ void __launch_bounds__(256) gru_fwd_persist_kernel(GruPersistArgs a) {
+  constexpr int NKB = HP / 16, NW = HP / 32;
+  __shared__ __align__(16) f32x4 tile[2][HP / 4 * kPt];  // h_{t-1}; r h_{t-1}
+  __shared__ __align__(16) f32x4 red[2][4][kPt][kPt / 4 + 1];  // [z, r | n][wave][unit][samples]
+  __shared__ int place[2];
+  const int H = a.H, B = a.B, S = a.S, NUT = (H + kPt - 1) / kPt, units = NUT * kPt;
+  int st, ut;
+  if (!persist_place(a.sync, NUT, st, ut, place)) return;
+  if (st >= a.nst) return;
+  const int64_t BS = (int64_t)B * S;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, r = lane & 15;
+  const int b0 = st * kPt, j0 = ut * kPt;
+  // z (waves 0, 2) and r (1, 3): half of the k-blocks each; n: a quarter per wave
+  f32x4 wzr[NKB / 2], wn[NKB / 4];
+  auto weight = [&](int k, int gate) {
+    return k < H && j0 + r < H ? a.W_hh[k + (int64_t)H * ((int64_t)gate * H + j0 + r)] : 0.f;
+  };
+  const int kz = (wave >> 1) * (NKB / 2), kn = wave * (NKB / 4);
+#pragma unroll
+  for (int k = 0; k < NKB / 2; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wzr[k][e] = weight(16 * (kz + k) + 4 * q + e, wave & 1);
+#pragma unroll
+  for (int k = 0; k < NKB / 4; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wn[k][e] = weight(16 * (kn + k) + 4 * q + e, 2);
+  // cell thread: sample m, unit u
+  const int m = tid & 15, u = tid >> 4;
+  const int64_t n = b0 + m, d = j0 + u;
+  const bool in = n < B && d < H;
+  const float bz = in ? a.bias[d] : 0.f, br = in ? a.bias[d + H] : 0.f, bn = in ? a.bias[d + 2 * H] : 0.f;
+  const unsigned slot = (unsigned)a.nst * units * kPt * 8u;  // bytes of one slot of one area
+  u64* const mine = a.ex + ((int64_t)st * units + d) * kPt + m;
+  const __amdgpu_buffer_rsrc_t rs = ex_rsrc(a.ex + (int64_t)st * units * kPt);
+  float* g = a.gates + n;
+  float xz = 0.f, xr = 0.f, xn = 0.f, hp = 0.f;
+  if (in) {
+    xz = g[BS * d];
+    xr = g[BS * (d + H)];
+    xn = g[BS * (d + 2 * H)];
+  }
+  const float* redf = reinterpret_cast<const float*>(red);
+  auto part = [&](int which, int w) { return redf[((which * 4 + w) * kPt + u) * (kPt + 4) + m]; };
+  for (int t = 0; t < S; ++t) {
+    float hz = 0.f, hr = 0.f, pn = 0.f;
+    if (t > 0) {
+      u32x4 w[NW];
+      const unsigned soff = ((t - 1) & 1) * slot, stamp = ex_stamp(a.sync, t);
+      gru_gather_issue<NW, kFirstPollSleep>(rs, soff, stamp, units, w);
+      const bool ok = ex_finish<NW, 4096>(a.sync, rs, tid * 16u, soff, stamp, w);
+      gru_stage(tile[0], w);
+      if (__syncthreads_or(!ok)) return;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      gru_product(tile[0], kz, wzr, acc);
+      red[0][wave][r][q] = acc;
+      __syncthreads();
+      hz = part(0, 0) + part(0, 2);
+      hr = part(0, 1) + part(0, 3);
+    }
+    const float zg = sigm((xz + hz) + bz), rg = sigm((xr + hr) + br), rhv = in ? rg * hp : 0.f;
+    if (t > 0) {
+      ex_store(mine + (2 + (t & 1)) * (slot / 8), ex_word(rhv, ex_stamp(a.sync, t + 1)));
+      u32x4 w[NW];
+      const unsigned soff = (2 + (t & 1)) * slot, stamp = ex_stamp(a.sync, t + 1);
+      gru_gather_issue<NW, kFirstPollSleep>(rs, soff, stamp, units, w);
+      const bool ok = ex_finish<NW, 4096>(a.sync, rs, tid * 16u, soff, stamp, w);
+      gru_stage(tile[1], w);
+      if (__syncthreads_or(!ok)) return;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      gru_product(tile[1], kn, wn, acc);
+      red[1][wave][r][q] = acc;
+      __syncthreads();
+      pn = (part(1, 0) + part(1, 1)) + (part(1, 2) + part(1, 3));
+    }
+    const float nc = tanhf((xn + pn) + bn);
+    const float h = in ? (1.0f - zg) * nc + zg * hp : 0.f;
+    if (t + 1 < S) ex_store(mine + (t & 1) * (slot / 8), ex_word(h, ex_stamp(a.sync, t + 1)));
+    if (in) {
+      const int64_t row = (int64_t)B * t;
+      g[row + BS * d] = zg;
+      g[row + BS * (d + H)] = rg;
+      g[row + BS * (d + 2 * H)] = nc;
+      a.rh[n + row + BS * d] = rhv;
+      a.Y[n + row + BS * d] = h;
+      if (t + 1 < S) {
+        xz = g[row + B + BS * d];
+        xr = g[row + B + BS * (d + H)];
+        xn = g[row + B + BS * (d + 2 * H)];
+      }
+    }
+    hp = h;
+  }
+}
+
+// Backward through time (gru_bwd_a_kernel / gru_bwd_b_kernel's arithmetic):
+// each step hands on dn and dz, forms d_rh = dn W_hn^T for its units from
+// everyone's dn, hands on dr, and forms dh_{t-1} = dh z + d_rh r + dz W_hz^T
+// + dr W_hr^T (the dz part while dr arrives).
+template <int HP>
+__global__ void __launch_bounds__(256) gru_bwd_persist_kernel(GruPersistArgs a) {
+  constexpr int NKB = HP / 16, NW = HP / 32, NQ = NKB / 4;
+  __shared__ __align__(16) f32x4 tile[2][HP / 4 * kPt];  // dn, then dr; dz
+  __shared__ __align__(16) f32x4 red[2][4][kPt][kPt / 4 + 1];
+  __shared__ int place[2];
+  const int H = a.H, B = a.B, S = a.S, NUT = (H + kPt - 1) / kPt, units = NUT * kPt;
+  int st, ut;
+  if (!persist_place(a.sync, NUT, st, ut, place)) return;
+  if (st >= a.nst) return;
+  const int64_t BS = (int64_t)B * S;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, r = lane & 15;
+  const int b0 = st * kPt, j0 = ut * kPt, k0 = wave * NQ;
+  // W_hh(unit j0 + r, column gate H + k): the transposed products' weights
+  f32x4 wz[NQ], wr[NQ], wn[NQ];
+#pragma unroll
+  for (int k = 0; k < NQ; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int c = 16 * (k0 + k) + 4 * q + e;
+      const bool ok = c < H && j0 + r < H;
+      const float* p = a.W_hh + (j0 + r) + (int64_t)H * c;
+      wz[k][e] = ok ? p[0] : 0.f;
+      wr[k][e] = ok ? p[(int64_t)H * H] : 0.f;
+      wn[k][e] = ok ? p[(int64_t)2 * H * H] : 0.f;
+    }
+  const int m = tid & 15, u = tid >> 4;
+  const int64_t n = b0 + m, d = j0 + u;
+  const bool in = n < B && d < H;
+  const unsigned slot = (unsigned)a.nst * units * kPt * 8u;
+  u64* const mine = a.ex + ((int64_t)st * units + d) * kPt + m;
+  const __amdgpu_buffer_rsrc_t rs = ex_rsrc(a.ex + (int64_t)st * units * kPt);
+  const float* redf = reinterpret_cast<const float*>(red);
+  auto sum = [&](int which) {
+    auto part = [&](int w) { return redf[((which * 4 + w) * kPt + u) * (kPt + 4) + m]; };
+    return (part(0) + part(1)) + (part(2) + part(3));
+  };
+  float dh = 0.f, zg = 0.f, rg = 0.f, nc = 0.f, hp = 0.f, dy = 0.f;
+  auto fetch = [&](int t) {
+    if (!in) return;
+    const int64_t row = n + (int64_t)B * t;
+    zg = a.gates[row + BS * d];
+    rg = a.gates[row + BS * (d + H)];
+    nc = a.gates[row + BS * (d + 2 * H)];
+    hp = t > 0 ? a.Y[row - B + BS * d] : 0.f;
+    dy = a.dY[row + BS * d];
+  };
+  fetch(S - 1);
+  for (int t = S - 1; t >= 0; --t) {
+    const unsigned par = (unsigned)(t & 1), stamp = ex_stamp(a.sync, S - t);
+    const float dhv = dy + dh;
+    const float dn = (dhv * (1.0f - zg)) * (1.0f - nc * nc);
+    const float dz = (dhv * (hp - nc)) * zg * (1.0f - zg);
+    ex_store(mine + par * (slot / 8), ex_word(in ? dn : 0.f, stamp));
+    if (t > 0) ex_store(mine + (2 + par) * (slot / 8), ex_word(in ? dz : 0.f, stamp));
+    const int64_t row = n + (int64_t)B * t;
+    if (in) {
+      a.dG[row + BS * d] = dz;
+      a.dG[row + BS * (d + 2 * H)] = dn;
+    }
+    u32x4 w[NW];
+    gru_gather_issue<NW, kFirstPollSleep>(rs, par * slot, stamp, units, w);
+    bool ok = ex_finish<NW, 4096>(a.sync, rs, tid * 16u, par * slot, stamp, w);
+    gru_stage(tile[0], w);
+    if (t > 0) gru_gather_issue<NW, 0>(rs, (2 + par) * slot, stamp, units, w);  // sent with dn
+    if (__syncthreads_or(!ok)) return;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    gru_product(tile[0], k0, wn, acc);
+    red[0][wave][r][q] = acc;
+    __syncthreads();
+    const float drh = sum(0);
+    const float dr = (drh * hp) * rg * (1.0f - rg);
+    const float part = dhv * zg + drh * rg;
+    if (in) a.dG[row + BS * (d + H)] = dr;
+    if (t == 0) break;
+    ex_store(mine + (4 + par) * (slot / 8), ex_word(in ? dr : 0.f, stamp));
+    fetch(t - 1);
+    ok = ex_finish<NW, 4096>(a.sync, rs, tid * 16u, (2 + par) * slot, stamp, w);
+    gru_stage(tile[1], w);
+    if (__syncthreads_or(!ok)) return;
+    gru_gather_issue<NW, 0>(rs, (4 + par) * slot, stamp, units, w);
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    gru_product(tile[1], k0, wz, acc);
+    ok = ex_finish<NW, 4096>(a.sync, rs, tid * 16u, (4 + par) * slot, stamp, w);
+    gru_stage(tile[0], w);  // every wave has read dn: two barriers ago
+    if (__syncthreads_or(!ok)) return;
+    gru_product(tile[0], k0, wr, acc);
+    red[1][wave][r][q] = acc;
+    __syncthreads();
+    dh = sum(1) + part;
+  }
+}
+
 // ---------------------------------------------------------------- GRU cells
 // gru.cpp:102-109: z, r from x W_ih + h W_hh (+ b); rh = r * h_prev.
 // hz: [B, 2H] dense = h_{t-1} W_hh[:, 0:2H] (ignored at t = 0, where h = 0).
@@ -1664,6 +1931,37 @@ int lstm_fwd_persistent(float* gates, const float* b, float* c, float* tanh_c, f
   return CNHIP_OK;
 }
 
+// The GRU recurrence (forward or BPTT) in one persistent launch where the
+// shape suits it; false in *done to fall back to the per-step launches: a
+// single step, H past 512, or more blocks than the chip holds at once.
+template <int HP>
+const void* gru_kernel(bool fwd) {
+  return fwd ? reinterpret_cast<const void*>(&gru_fwd_persist_kernel<HP>)
+             : reinterpret_cast<const void*>(&gru_bwd_persist_kernel<HP>);
+}
+int gru_persistent(bool fwd, GruPersistArgs args, int64_t B, int64_t S, int64_t H, hipStream_t st, const char* who,
+                   bool* done) {
+  *done = false;
+  if (!persist_enabled() || S < 2 || S > 65000 || H > kPersistMaxH || B * S * 3 * H > INT32_MAX) return CNHIP_OK;
+  const void* kern = H <= 64    ? gru_kernel<64>(fwd)
+                     : H <= 128 ? gru_kernel<128>(fwd)
+                     : H <= 256 ? gru_kernel<256>(fwd)
+                                : gru_kernel<512>(fwd);
+  const int64_t nst = (B + kPt - 1) / kPt, nut = (H + kPt - 1) / kPt, grid = 8 * nut * ((nst + 7) / 8);
+  const size_t ex_bytes = (size_t)(fwd ? 4 : 6) * nst * nut * kPt * kPt * sizeof(u64);
+  if (ex_bytes > 0x7fffffffu || !persist_fits(kern, grid, 256, who)) return CNHIP_OK;
+  args.B = (int)B;
+  args.S = (int)S;
+  args.H = (int)H;
+  args.nst = (int)nst;
+  TimingRec* rec = timing_slot(2.0 * B * 3 * H * H * (double)(S - 1));
+  if (rec) (void)hipEventRecord(rec->start, st);
+  CNHIP_TRY(persist_launch(kern, grid, 256, args, ex_bytes, st, who));
+  if (rec) (void)hipEventRecord(rec->stop, st);
+  *done = true;
+  return CNHIP_OK;
+}
+
 int check_rnn(int64_t B, int64_t S, int64_t I, int64_t H, const char* who) {
   CNHIP_REQUIRE(B > 0 && S > 0 && I > 0 && H > 0, "%s: bad shape B=%lld S=%lld I=%lld H=%lld", who,
                 (long long)B, (long long)S, (long long)I, (long long)H);
@@ -1801,6 +2099,7 @@ int cnhip_gru_forward(const float* X, const float* W_ih, const float* W_hh, cons
   CNHIP_TRY(cnhip::check_rnn(B, S, I, H, who));
   CNHIP_REQUIRE(X && W_ih && W_hh && b && Y && gates && rh, "%s: NULL pointer", who);
   hipStream_t st = as_stream(stream);
+  CNHIP_TRY(cnhip::recurrence_fault_check(st, who));
   const int64_t G = 3 * H, BS = B * S;
   cnhip::Workspace ws(st);
   CNHIP_TRY(ws.alloc((size_t)(3 * B * H) * sizeof(float), who));
@@ -1808,6 +2107,15 @@ int cnhip_gru_forward(const float* X, const float* W_ih, const float* W_hh, cons
   float* proj = hz + 2 * B * H;           // [B, H]
   const float* W_hn = W_hh + H * 2 * H;
   CNHIP_TRY(cnhip::gemm_f32(0, 0, BS, G, I, 1.f, X, BS, W_ih, I, 0.f, gates, BS, nullptr, 0, st, who));
+  cnhip::GruPersistArgs args{};
+  args.gates = gates;
+  args.bias = b;
+  args.Y = Y;
+  args.rh = rh;
+  args.W_hh = W_hh;
+  bool done = false;
+  CNHIP_TRY(cnhip::gru_persistent(true, args, B, S, H, st, who, &done));
+  if (done) return CNHIP_OK;
   for (int64_t t = 0; t < S; ++t) {
     if (t > 0)
       CNHIP_TRY(cnhip::gemm_f32(0, 0, B, 2 * H, H, 1.f, Y + B * (t - 1), BS, W_hh, H, 0.f, hz, B,
@@ -1833,6 +2141,7 @@ int cnhip_gru_backward(const float* X, const float* W_ih, const float* W_hh, con
   CNHIP_REQUIRE(X && W_ih && W_hh && Y && gates && rh && dY && gW_ih && gW_hh && gb,
                 "%s: NULL pointer", who);
   hipStream_t st = as_stream(stream);
+  CNHIP_TRY(cnhip::recurrence_fault_check(st, who));
   const int64_t G = 3 * H, BS = B * S;
   cnhip::Workspace ws(st);
   CNHIP_TRY(ws.alloc((size_t)(BS * G + 2 * B * H) * sizeof(float), who));
@@ -1840,7 +2149,15 @@ int cnhip_gru_backward(const float* X, const float* W_ih, const float* W_hh, con
   float* dh = dG + BS * G;
   float* drh = dh + B * H;
   const float* W_hn = W_hh + H * 2 * H;
-  for (int64_t t = S - 1; t >= 0; --t) {
+  cnhip::GruPersistArgs args{};
+  args.gates = const_cast<float*>(gates);
+  args.Y = const_cast<float*>(Y);
+  args.dY = dY;
+  args.dG = dG;
+  args.W_hh = W_hh;
+  bool done = false;
+  CNHIP_TRY(cnhip::gru_persistent(false, args, B, S, H, st, who, &done));
+  for (int64_t t = done ? -1 : S - 1; t >= 0; --t) {
     hipLaunchKernelGGL(cnhip::gru_bwd_a_kernel, dim3(cnhip::cell_grid(B, H)), dim3(256), 0, st,
                        gates, Y, dY, dh, dG, B, S, H, t, t == S - 1 ? 1 : 0);
     CNHIP_TRY(cnhip::check_launch(who));
