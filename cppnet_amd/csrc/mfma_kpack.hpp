@@ -33,6 +33,8 @@ namespace kp {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// a float4 at any 4-byte-aligned address (global_load/store_dwordx4 take it)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int WGM_, int WGN_, int WM_, int WN_, int BK_ = 16, int WGK_ = 1>
 struct Cfg {
@@ -88,8 +90,9 @@ struct Operand {
     return true;
   }
 
-  // FAST: the whole tile is in range and 16-byte aligned.  Otherwise every
-  // element is bounds-checked (rows < Rtot, k < Kend) and zero-filled.
+  // FAST: the whole tile is in range and 16-byte aligned.  Otherwise a unit
+  // in range is one float4 load at any alignment, and the elements of the
+  // others are bounds-checked (rows < Rtot, k < Kend) and zero-filled.
   template <bool FAST>
   __device__ __forceinline__ static void load(const float* __restrict__ X, int64_t ld, int64_t r0,
                                               int64_t k0, int64_t Rtot, int64_t Kend,
@@ -103,6 +106,10 @@ struct Operand {
         v[p] = *reinterpret_cast<const f32x4*>(X + (KC ? gk + ld * gr : gr + ld * gk));
       } else {
         f32x4 t;
+        if (KC ? (gr < Rtot && gk + 3 < Kend) : (gr + 3 < Rtot && gk < Kend)) {
+          v[p] = *reinterpret_cast<const f32x4u*>(X + (KC ? gk + ld * gr : gr + ld * gk));
+          continue;
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const bool in = KC ? (gr < Rtot && gk + j < Kend) : (gr + j < Rtot && gk < Kend);

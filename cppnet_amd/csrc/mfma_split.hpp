@@ -43,8 +43,7 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-// a float4 at any 4-byte-aligned address (global_load/store_dwordx4 take it)
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+using kp::f32x4u;
 
 constexpr int KT = 16;  // k-tile depth: one MFMA step
 
