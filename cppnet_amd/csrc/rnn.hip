@@ -1322,6 +1322,183 @@ __global__ void __launch_bounds__(256) gru_bwd_persist_kernel(GruPersistArgs a) 
   }
 }
 
+// ---------------------------------------------------------------- persistent LSTM, any size
+// The LSTM recurrence for the batches and hidden sizes that the tuned
+// persistent kernels above do not take (B no multiple of 16, H not 64, 128,
+// 256 or 512), in the manner of the persistent GRU: rows past B and units
+// past H are zeros.  Wave w owns gate w of the block's 16 units in both
+// passes: forward h_{t-1} W_hh for its 16 columns, backward dG_gate W_hh^T
+// for the 16 units, so each block gathers all four gate gradients.  The
+// input projection and the weight gradients stay GEMMs.  Bound by the
+// hand-over of a step, as the others; per step and pass the launches this
+// replaces took 8-9 us.
+struct LstmAnyArgs {
+  float* gates;
+  const float* bias;
+  float* c;
+  float* tanh_c;
+  float* Y;
+  const float* dY;
+  float* dG;
+  const float* W_hh;
+  u64* ex;  // areas of [2 slots][nst][NUT 16][16] words: h, or the four gate gradients
+  int B, S, H, nst, dy_last;
+  PersistSync sync;
+};
+
+template <int HP>
+__global__ void __launch_bounds__(256) lstm_fwd_any_kernel(LstmAnyArgs a) {
+  constexpr int NKB = HP / 16, NW = HP / 32;
+  __shared__ __align__(16) f32x4 tile[HP / 4 * kPt];
+  __shared__ __align__(16) f32x4 red[4][kPt][kPt / 4 + 1];  // [gate][unit][samples]
+  __shared__ int place[2];
+  const int H = a.H, B = a.B, S = a.S, NUT = (H + kPt - 1) / kPt, units = NUT * kPt;
+  int st, ut;
+  if (!persist_place(a.sync, NUT, st, ut, place)) return;
+  if (st >= a.nst) return;
+  const int64_t BS = (int64_t)B * S;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, r = lane & 15;
+  const int b0 = st * kPt, j0 = ut * kPt;
+  f32x4 wv[NKB];
+#pragma unroll
+  for (int k = 0; k < NKB; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int kk = 16 * k + 4 * q + e;
+      wv[k][e] = kk < H && j0 + r < H ? a.W_hh[kk + (int64_t)H * ((int64_t)wave * H + j0 + r)] : 0.f;
+    }
+  const int m = tid & 15, u = tid >> 4;
+  const int64_t n = b0 + m, d = j0 + u;
+  const bool in = n < B && d < H;
+  const unsigned slot = (unsigned)a.nst * units * kPt * 8u;
+  u64* const mine = a.ex + ((int64_t)st * units + d) * kPt + m;
+  const __amdgpu_buffer_rsrc_t rs = ex_rsrc(a.ex + (int64_t)st * units * kPt);
+  float* g = a.gates + n;
+  float x[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f}, c_prev = 0.f;
+  if (in) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      x[k] = g[BS * (d + (int64_t)k * H)];
+      b[k] = a.bias[d + (int64_t)k * H];
+    }
+  }
+  const float* redf = reinterpret_cast<const float*>(red);
+  for (int t = 0; t < S; ++t) {
+    float p[4] = {0.f, 0.f, 0.f, 0.f};
+    if (t > 0) {
+      u32x4 w[NW];
+      const unsigned soff = ((t - 1) & 1) * slot, stamp = ex_stamp(a.sync, t);
+      gru_gather_issue<NW, kFirstPollSleep>(rs, soff, stamp, units, w);
+      const bool ok = ex_finish<NW, 4096>(a.sync, rs, tid * 16u, soff, stamp, w);
+      gru_stage(tile, w);
+      if (__syncthreads_or(!ok)) return;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      gru_product(tile, 0, wv, acc);
+      red[wave][r][q] = acc;
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < 4; ++k) p[k] = redf[(k * kPt + u) * (kPt + 4) + m];
+    }
+    const float ig = sigm((p[0] + x[0]) + b[0]), fg = sigm((p[1] + x[1]) + b[1]);
+    const float gg = tanhf((p[2] + x[2]) + b[2]), og = sigm((p[3] + x[3]) + b[3]);
+    const float ct = lstm_cell_c(fg, c_prev, ig, gg), tc = tanhf(ct);
+    const float h = in ? og * tc : 0.f;
+    if (t + 1 < S) ex_store(mine + (t & 1) * (slot / 8), ex_word(h, ex_stamp(a.sync, t + 1)));
+    if (in) {
+      const int64_t row = (int64_t)B * t;
+      g[row + BS * d] = ig;
+      g[row + BS * (d + H)] = fg;
+      g[row + BS * (d + 2 * (int64_t)H)] = gg;
+      g[row + BS * (d + 3 * (int64_t)H)] = og;
+      a.c[n + row + BS * d] = ct;
+      a.tanh_c[n + row + BS * d] = tc;
+      a.Y[n + row + BS * d] = h;
+      if (t + 1 < S) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = g[row + B + BS * (d + (int64_t)k * H)];
+      }
+    }
+    c_prev = ct;
+  }
+}
+
+template <int HP>
+__global__ void __launch_bounds__(256) lstm_bwd_any_kernel(LstmAnyArgs a) {
+  constexpr int NKB = HP / 16, NW = HP / 32;
+  __shared__ __align__(16) f32x4 tile[4][HP / 4 * kPt];
+  __shared__ __align__(16) f32x4 red[4][kPt][kPt / 4 + 1];
+  __shared__ int place[2];
+  const int H = a.H, B = a.B, S = a.S, NUT = (H + kPt - 1) / kPt, units = NUT * kPt;
+  int st, ut;
+  if (!persist_place(a.sync, NUT, st, ut, place)) return;
+  if (st >= a.nst) return;
+  const int64_t BS = (int64_t)B * S;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, r = lane & 15;
+  const int b0 = st * kPt, j0 = ut * kPt;
+  f32x4 wv[NKB];  // W_hh(unit j0 + r, column wave H + k)
+#pragma unroll
+  for (int k = 0; k < NKB; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int kk = 16 * k + 4 * q + e;
+      wv[k][e] = kk < H && j0 + r < H ? a.W_hh[(j0 + r) + (int64_t)H * ((int64_t)wave * H + kk)] : 0.f;
+    }
+  const int m = tid & 15, u = tid >> 4;
+  const int64_t n = b0 + m, d = j0 + u;
+  const bool in = n < B && d < H;
+  const unsigned slot = (unsigned)a.nst * units * kPt * 8u;
+  u64* const mine = a.ex + ((int64_t)st * units + d) * kPt + m;
+  const __amdgpu_buffer_rsrc_t rs = ex_rsrc(a.ex + (int64_t)st * units * kPt);
+  const float* redf = reinterpret_cast<const float*>(red);
+  float dh = 0.f, dc = 0.f, ig = 0.f, fg = 0.f, gg = 0.f, og = 0.f, tc = 0.f, cprev = 0.f, dy = 0.f;
+  auto fetch = [&](int t) {
+    if (!in) return;
+    const int64_t row = n + (int64_t)B * t;
+    ig = a.gates[row + BS * d];
+    fg = a.gates[row + BS * (d + H)];
+    gg = a.gates[row + BS * (d + 2 * (int64_t)H)];
+    og = a.gates[row + BS * (d + 3 * (int64_t)H)];
+    tc = a.tanh_c[row + BS * d];
+    cprev = t > 0 ? a.c[row - B + BS * d] : 0.f;
+    if (!a.dy_last) dy = a.dY[row + BS * d];
+    else dy = t == S - 1 ? a.dY[n + (int64_t)B * d] : 0.f;
+  };
+  fetch(S - 1);
+  for (int t = S - 1; t >= 0; --t) {
+    const unsigned par = (unsigned)(t & 1), stamp = ex_stamp(a.sync, S - t);
+    float dg[4], dcn;
+    lstm_cell_bwd(ig, fg, gg, og, tc, dy + dh, dc, cprev, dg[0], dg[1], dg[2], dg[3], dcn);
+    dc = dcn;
+    const int64_t row = n + (int64_t)B * t;
+    if (t > 0) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) ex_store(mine + (2 * k + par) * (slot / 8), ex_word(in ? dg[k] : 0.f, stamp));
+    }
+    if (in) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) a.dG[row + BS * (d + (int64_t)k * H)] = dg[k];
+    }
+    if (t == 0) break;
+    fetch(t - 1);
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      u32x4 w[NW];
+      if (k == 0) gru_gather_issue<NW, kFirstPollSleep>(rs, par * slot, stamp, units, w);
+      else gru_gather_issue<NW, 0>(rs, (2 * k + par) * slot, stamp, units, w);
+      ok = ok && ex_finish<NW, 4096>(a.sync, rs, tid * 16u, (2 * k + par) * slot, stamp, w);
+      gru_stage(tile[k], w);
+    }
+    if (__syncthreads_or(!ok)) return;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    gru_product(tile[wave], 0, wv, acc);
+    red[wave][r][q] = acc;
+    __syncthreads();
+    auto part = [&](int w) { return redf[(w * kPt + u) * (kPt + 4) + m]; };
+    dh = (part(0) + part(1)) + (part(2) + part(3));
+  }
+}
+
 // ---------------------------------------------------------------- GRU cells
 // gru.cpp:102-109: z, r from x W_ih + h W_hh (+ b); rh = r * h_prev.
 // hz: [B, 2H] dense = h_{t-1} W_hh[:, 0:2H] (ignored at t = 0, where h = 0).
@@ -1962,6 +2139,37 @@ int gru_persistent(bool fwd, GruPersistArgs args, int64_t B, int64_t S, int64_t 
   return CNHIP_OK;
 }
 
+// The LSTM recurrence (forward or BPTT) of any B and any H up to 512 in one
+// persistent launch, where the chip holds its blocks; false in *done to fall
+// back to the per-step launches.
+template <int HP>
+const void* lstm_any_kernel(bool fwd) {
+  return fwd ? reinterpret_cast<const void*>(&lstm_fwd_any_kernel<HP>)
+             : reinterpret_cast<const void*>(&lstm_bwd_any_kernel<HP>);
+}
+int lstm_any_persistent(bool fwd, LstmAnyArgs args, int64_t B, int64_t S, int64_t H, hipStream_t st, const char* who,
+                        bool* done) {
+  *done = false;
+  if (!persist_enabled() || S < 2 || S > 65000 || H > kPersistMaxH || B * S * 4 * H > INT32_MAX) return CNHIP_OK;
+  const void* kern = H <= 64    ? lstm_any_kernel<64>(fwd)
+                     : H <= 128 ? lstm_any_kernel<128>(fwd)
+                     : H <= 256 ? lstm_any_kernel<256>(fwd)
+                                : lstm_any_kernel<512>(fwd);
+  const int64_t nst = (B + kPt - 1) / kPt, nut = (H + kPt - 1) / kPt, grid = 8 * nut * ((nst + 7) / 8);
+  const size_t ex_bytes = (size_t)(fwd ? 2 : 8) * nst * nut * kPt * kPt * sizeof(u64);
+  if (ex_bytes > 0x7fffffffu || !persist_fits(kern, grid, 256, who)) return CNHIP_OK;
+  args.B = (int)B;
+  args.S = (int)S;
+  args.H = (int)H;
+  args.nst = (int)nst;
+  TimingRec* rec = timing_slot(2.0 * B * 4 * H * H * (double)(S - 1));
+  if (rec) (void)hipEventRecord(rec->start, st);
+  CNHIP_TRY(persist_launch(kern, grid, 256, args, ex_bytes, st, who));
+  if (rec) (void)hipEventRecord(rec->stop, st);
+  *done = true;
+  return CNHIP_OK;
+}
+
 int check_rnn(int64_t B, int64_t S, int64_t I, int64_t H, const char* who) {
   CNHIP_REQUIRE(B > 0 && S > 0 && I > 0 && H > 0, "%s: bad shape B=%lld S=%lld I=%lld H=%lld", who,
                 (long long)B, (long long)S, (long long)I, (long long)H);
@@ -2002,6 +2210,17 @@ int lstm_backward(const float* X, const float* W_ih, const float* W_hh, const fl
   bool done = false, fused = false;
   CNHIP_TRY(lstm_bwd_persistent(gates, c, tanh_c, dY, dy_last, W_hh, dG, X, Y, part, I, gW_hh, gW_ih, gb, B, S, H,
                                 st, who, &done, &fused));
+  if (!done) {
+    LstmAnyArgs any{};
+    any.gates = const_cast<float*>(gates);
+    any.c = const_cast<float*>(c);
+    any.tanh_c = const_cast<float*>(tanh_c);
+    any.dY = dY;
+    any.dG = dG;
+    any.W_hh = W_hh;
+    any.dy_last = dy_last ? 1 : 0;
+    CNHIP_TRY(lstm_any_persistent(false, any, B, S, H, st, who, &done));
+  }
   if (!done) {
     const float* dYs = dY;
     if (dy_last) {
@@ -2068,6 +2287,15 @@ int cnhip_lstm_forward(const float* X, const float* W_ih, const float* W_hh, con
   if (done) return CNHIP_OK;
   CNHIP_TRY(cnhip::gemm_f32(0, 0, BS, G, I, 1.f, X, BS, W_ih, I, 0.f, gates, BS, nullptr, 0, st, who));
   CNHIP_TRY(cnhip::lstm_fwd_persistent(gates, b, c, tanh_c, Y, W_hh, X, W_ih, I, false, B, S, H, st, who, &done));
+  if (done) return CNHIP_OK;
+  cnhip::LstmAnyArgs any{};
+  any.gates = gates;
+  any.bias = b;
+  any.c = c;
+  any.tanh_c = tanh_c;
+  any.Y = Y;
+  any.W_hh = W_hh;
+  CNHIP_TRY(cnhip::lstm_any_persistent(true, any, B, S, H, st, who, &done));
   if (done) return CNHIP_OK;
   // t = 0: h_0 = 0, no recurrent term; then one fused GEMM + cell launch per step
   hipLaunchKernelGGL(cnhip::lstm_cell_fwd0_kernel, dim3(cnhip::cell_grid(B, H)), dim3(256), 0, st,
