@@ -307,7 +307,8 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& g, float* lds, int bx
     const bool tiny =
         T::run(A, g.lda, B, g.ldb, g.M, g.N, m0, n0, k_begin, k_end, reinterpret_cast<char*>(lds), park, split & 1, acc);
     if (C::WGK > 1 && threadIdx.x >= C::NT / C::WGK) return;  // group 0 holds the sums
-    if (T::needs_fp32(acc, tiny)) T::fp32(A, g.lda, B, g.ldb, g.M, g.N, m0, n0, k_begin, k_end, acc);
+    if (T::needs_fp32(acc, tiny) || (tiny && T::large(A, g.lda, B, g.ldb, g.M, g.N, m0, n0, k_begin, k_end)))
+      T::fp32(A, g.lda, B, g.ldb, g.M, g.N, m0, n0, k_begin, k_end, acc);
   } else {
     const bool fast = g.vec_ok && full_mn && ((k_end - k_begin) % C::BK == 0);
     if (fast) gemm_mainloop<true, TA, TB, C>(g, A, B, m0, n0, k_begin, k_end, lds, acc);

@@ -21,10 +21,15 @@
 // (positive) of the fp32 MFMA's.
 //
 // What bf16 terms cannot hold is caught per wave after the contraction
-// (needs_fp32 below) and that wave's outputs are formed again with fp32 MFMAs
-// straight from memory: infinities and NaN (inf = inf + NaN + NaN would turn
-// an infinite product into NaN), values whose bf16 rounding overflows, and
-// values below 2^-100, whose low terms the matrix cores flush to zero.
+// (needs_fp32 and large below) and that wave's outputs are formed again with
+// fp32 MFMAs straight from memory: infinities and NaN (inf = inf + NaN + NaN
+// would turn an infinite product into NaN), values whose bf16 rounding
+// overflows, and values below 2^-100, whose low terms the matrix cores flush
+// to zero, where an output is below 2^-60 or another operand value is 2^30
+// or more, and products whose low terms it flushes, where an output is
+// nonzero and below 2^-84.  Otherwise what is lost of an operand, 2 * 2^-126
+// * 2^30 a product, is below 2^-24 of every output for contractions up to
+// 2^11 terms of one sign or 2^22 of mixed signs.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -454,10 +459,11 @@ struct Tile {
 
   // Whether this wave's outputs have to be formed with fp32 MFMAs: one is not
   // finite (an operand was not, or its bf16 term overflowed), or one is below
-  // 2^-60 while some operand element was below 2^-100, so that low terms
-  // flushed to zero could be a part of it that counts.
+  // 2^-60 while some operand element was below 2^-100, or one is nonzero and
+  // below 2^-84, so that terms flushed to zero could be a part of it that
+  // counts.
   __device__ __forceinline__ static bool needs_fp32(const f32x16 (&acc)[C::WM][C::WN], bool tiny) {
-    float hi = 0.f, lo = INFINITY;
+    float hi = 0.f, lo = INFINITY, lo_nz = INFINITY;
     bool nan = false;
 #pragma unroll
     for (int i = 0; i < C::WM; ++i)
@@ -469,20 +475,20 @@ struct Tile {
           nan |= x != x;
           hi = fmaxf(hi, fabsf(x));
           lo = fminf(lo, fabsf(x));
+          lo_nz = fminf(lo_nz, x == 0.f ? INFINITY : fabsf(x));
         }
-    const bool bad = nan || hi == INFINITY || (tiny && lo < 0x1p-60f);
+    const bool bad = nan || hi == INFINITY || (tiny && lo < 0x1p-60f) || lo_nz < 0x1p-84f;
     return __any(bad);
   }
 
-  // The wave's outputs with v_mfma_f32_32x32x2f32, operands straight from
-  // memory: slow, for the rare waves that needs_fp32 names.
-  __device__ __forceinline__ static void fp32(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
-                                           int64_t N, int64_t m0, int64_t n0, int64_t k_begin, int64_t k_end,
-                                           f32x16 (&acc)[C::WM][C::WN]) {
+  // f(a, b): the wave's operand values at k, k + 1, straight from memory
+  // (zeros past the edges), over the whole contraction.
+  template <class F>
+  __device__ __forceinline__ static void each_k(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
+                                             int64_t N, int64_t m0, int64_t n0, int64_t k_begin, int64_t k_end, F&& f) {
     int wm, wn, wk;
     kp::wave_pos<C>(wm, wn, wk);
     const int lane = threadIdx.x & 63, h = lane >> 5, r = lane & 31;
-    kp::zero_acc<C>(acc);
     for (int64_t k = k_begin; k < k_end; k += 2) {
       const int64_t kk = k + h;
       float a[C::WM], b[C::WN];
@@ -496,12 +502,39 @@ struct Tile {
         const int64_t n = n0 + wn * (C::WN * 32) + 32 * j + r;
         b[j] = n < N && kk < k_end ? B[!TB ? kk + ldb * n : n + ldb * kk] : 0.f;
       }
+      f(a, b);
+    }
+  }
+
+  // Whether this wave's operands hold a value of 2^30 or more: beside a
+  // flushed low term (below 2^-126) it can count in an output above 2^-60.
+  // Only asked where some element was below 2^-100, so it costs the others
+  // nothing.
+  __device__ __forceinline__ static bool large(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
+                                            int64_t N, int64_t m0, int64_t n0, int64_t k_begin, int64_t k_end) {
+    float hi = 0.f;
+    each_k(A, lda, B, ldb, M, N, m0, n0, k_begin, k_end, [&](const float (&a)[C::WM], const float (&b)[C::WN]) {
+#pragma unroll
+      for (int i = 0; i < C::WM; ++i) hi = fmaxf(hi, fabsf(a[i]));
+#pragma unroll
+      for (int j = 0; j < C::WN; ++j) hi = fmaxf(hi, fabsf(b[j]));
+    });
+    return __any(hi >= 0x1p30f);
+  }
+
+  // The wave's outputs with v_mfma_f32_32x32x2f32: slow, for the rare waves
+  // that needs_fp32 or large names.
+  __device__ __forceinline__ static void fp32(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
+                                           int64_t N, int64_t m0, int64_t n0, int64_t k_begin, int64_t k_end,
+                                           f32x16 (&acc)[C::WM][C::WN]) {
+    kp::zero_acc<C>(acc);
+    each_k(A, lda, B, ldb, M, N, m0, n0, k_begin, k_end, [&](const float (&a)[C::WM], const float (&b)[C::WN]) {
 #pragma unroll
       for (int i = 0; i < C::WM; ++i)
 #pragma unroll
         for (int j = 0; j < C::WN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
+    });
   }
 };
 

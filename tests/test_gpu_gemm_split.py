@@ -89,6 +89,28 @@ def test_gemm_split_nonfinite_and_range_ends(gpu, M, N, K):
     assert bool(((got - want).abs()[ok] <= lim[ok]).all()), float(((got - want).abs()[ok] / lim[ok]).max())
 
 
+@pytest.mark.parametrize("scale", [(-116, 122), (-58, -58)])
+@pytest.mark.parametrize("M,N,K", [(65, 80, 700), (300, 515, 785), (4096, 4096, 2048)])
+def test_gemm_split_terms_that_flush(gpu, M, N, K, scale):
+    """Ordinary outputs of values whose low bf16 terms are flushed, and outputs
+    so small that products of low terms are."""
+    gen = torch.Generator("cuda").manual_seed(M)
+    A = torch.randn(K, M, generator=gen, device="cuda")
+    B = torch.randn(N, K, generator=gen, device="cuda")
+    sa, sb = 2.0 ** scale[0], 2.0 ** scale[1]
+    if scale[1] > 0:
+        A[K // 2] *= sa
+        B[:, K // 2] *= sb
+    else:
+        A *= sa
+        B *= sb
+    C = torch.empty(N, M, device="cuda")
+    ops.gemm(False, False, M, N, K, A, M, B, K, C, M)
+    want = B.double() @ A.double()
+    size = (B.double().square() @ A.double().square()).sqrt()
+    assert bool(((C.double() - want).abs() <= 8 * 2.0 ** -24 * (K / 2) ** 0.5 * size + K * 2.0 ** -149).all())
+
+
 def test_linear_residual_in_place(gpu):
     """The skip branch added into its own buffer (Z is Y): a tile whose half
     sums would wait in C must not clobber it."""
