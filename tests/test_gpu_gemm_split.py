@@ -92,8 +92,8 @@ def test_gemm_split_nonfinite_and_range_ends(gpu, M, N, K):
 @pytest.mark.parametrize("scale", [(-116, 122), (-58, -58)])
 @pytest.mark.parametrize("M,N,K", [(65, 80, 700), (300, 515, 785), (4096, 4096, 2048)])
 def test_gemm_split_terms_that_flush(gpu, M, N, K, scale):
-    """Ordinary outputs of values whose low bf16 terms are flushed, and outputs
-    so small that products of low terms are."""
+    """Ordinary outputs of values whose low bf16 terms fall below their grid, and
+    outputs so small that products of low terms are subnormal."""
     gen = torch.Generator("cuda").manual_seed(M)
     A = torch.randn(K, M, generator=gen, device="cuda")
     B = torch.randn(N, K, generator=gen, device="cuda")
@@ -109,6 +109,56 @@ def test_gemm_split_terms_that_flush(gpu, M, N, K, scale):
     want = B.double() @ A.double()
     size = (B.double().square() @ A.double().square()).sqrt()
     assert bool(((C.double() - want).abs() <= 8 * 2.0 ** -24 * (K / 2) ** 0.5 * size + K * 2.0 ** -149).all())
+
+
+def low_end(A, B, case):
+    """A [K, M] (A(m, k) at [k, m]) and B [N, K] moved to the low end of the
+    range: one k, every element, one row of A, or one row of A and one column
+    of B, which alone are small enough for products to be subnormal."""
+    kind, ea, eb = case
+    sa, sb = 2.0 ** ea, 2.0 ** eb
+    k = A.shape[0] // 2
+    if kind == "k":
+        A[k] *= sa
+        B[:, k] *= sb
+    elif kind == "all":
+        A *= sa
+        B *= sb
+    elif kind == "row":
+        A[:, 5] *= sa
+        B *= sb
+    else:
+        A[:, 5] *= sa
+        B[7] *= sb
+
+
+@pytest.mark.parametrize("case", [("k", -116, 122), ("k", -136, 126), ("k", -147, 127), ("all", -58, -58), ("all", -66, -66),
+                                  ("all", -100, -36), ("row", -140, 100), ("row", -120, 20), ("cross", -66, -66),
+                                  ("cross", -70, -72)], ids=str)
+@pytest.mark.parametrize("sign", ["mixed", "one"])
+@pytest.mark.parametrize("M,N,K", [(65, 80, 700), (300, 515, 785), (4096, 4096, 2048)])
+def test_gemm_split_low_end_of_the_range(gpu, M, N, K, case, sign):
+    """Operands whose low bits, or all of them, lie below the bf16 terms' grid,
+    and products that are subnormal."""
+    gen = torch.Generator("cuda").manual_seed(M)
+    A = torch.randn(K, M, generator=gen, device="cuda")
+    B = torch.randn(N, K, generator=gen, device="cuda")
+    if sign == "one":
+        A.abs_()
+        B.abs_()
+    # no product of one k overflows: |a b| < 2^126
+    A.clamp_(-4, 4)
+    low_end(A, B.clamp_(-1, 1) if case[0] == "k" else B, case)
+    C = torch.empty(N, M, device="cuda")
+    ops.gemm(False, False, M, N, K, A, M, B, K, C, M)
+    want = B.double() @ A.double()
+    size = (B.double().square() @ A.double().square()).sqrt()
+    # sums of one sign grow to sqrt(K) of that size; 2^-149: half of the
+    # smallest subnormal for each of K products
+    grow = 1 if sign == "mixed" else 0.5 * K ** 0.5
+    lim = 8 * 2.0 ** -24 * (K / 2) ** 0.5 * size * grow + K * 2.0 ** -149
+    err = (C.double() - want).abs()
+    assert bool((err <= lim).all()), f"worst error / bound {float((err / lim).max()):.3g}"
 
 
 def test_linear_residual_in_place(gpu):
