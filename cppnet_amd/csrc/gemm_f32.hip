@@ -304,10 +304,10 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& g, float* lds, int bx
   if constexpr (split_cfg<C>()) {
     using T = sp::Tile<TA, TB, C>;
     const sp::Park park{g.park ? g.C + batch * g.stride_c : nullptr, g.ldc, g.M, g.N, m0, n0};
-    const bool tiny =
+    const float least =
         T::run(A, g.lda, B, g.ldb, g.M, g.N, m0, n0, k_begin, k_end, reinterpret_cast<char*>(lds), park, split & 1, acc);
     if (C::WGK > 1 && threadIdx.x >= C::NT / C::WGK) return;  // group 0 holds the sums
-    if (T::needs_fp32(acc, tiny) || (tiny && T::large(A, g.lda, B, g.ldb, g.M, g.N, m0, n0, k_begin, k_end)))
+    if (T::needs_fp32(acc, least))
       T::fp32(A, g.lda, B, g.ldb, g.M, g.N, m0, n0, k_begin, k_end, acc);
   } else {
     const bool fast = g.vec_ok && full_mn && ((k_end - k_begin) % C::BK == 0);

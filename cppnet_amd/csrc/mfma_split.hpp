@@ -21,24 +21,23 @@
 // (positive) of the fp32 MFMA's.
 //
 // What bf16 terms cannot hold is caught per wave after the contraction
-// (needs_fp32 and large below) and that wave's outputs are formed again with
-// fp32 MFMAs straight from memory: infinities and NaN (inf = inf + NaN + NaN
-// would turn an infinite product into NaN), values whose bf16 rounding
-// overflows, and values near the low end of the range.  The matrix cores keep
-// subnormal bf16 inputs, products and sums (measured: 2^-70 * 2^-70 and
-// 2^-130 * 2^10 come back exact), but the terms themselves lie on a grid of
-// 2^-133, so a value below 2^-110 loses its low bits (2^-134 at most) and one
-// of 2^-134 or less all of them.  A wave is formed again where some nonzero
-// element of its block is below 2^-100 and an output is below 2^-60 or
-// another operand value is 2^30 or more: otherwise what is lost,
-// 2 * 2^-134 * 2^30 a product, is below 2^-24 of every output for
-// contractions up to 2^18 terms.  Outputs that are nonzero and below 2^-84
-// are formed again too.
+// (needs_fp32 below) and that wave's outputs are formed again with fp32 MFMAs
+// straight from memory: infinities and NaN (inf = inf + NaN + NaN would turn
+// an infinite product into NaN), values whose bf16 rounding overflows, and
+// values at the low end of the range.  The matrix cores keep subnormal bf16
+// inputs, products and sums (measured: 2^-70 * 2^-70 and 2^-130 * 2^10 come
+// back exact), but the terms themselves lie on a grid of 2^-133, so a value
+// below 2^-110 can lose up to 2^-134.  Where a block's operands hold such a
+// value, an output of the block is off by at most K 2^-133 times the largest
+// element, and a wave is formed again where that is more than 2^-24 of one of
+// its outputs (range, Tile::run).  Both bounds are kept while the operands are
+// staged, so nothing is read twice to find them.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "mfma_kpack.hpp"
 
@@ -55,18 +54,27 @@ using kp::f32x4u;
 
 constexpr int KT = 16;  // k-tile depth: one MFMA step
 
-// Two elements adjacent in k, split: w[p] holds term p of both, the lower k
-// in the low half.  tiny: running minimum over 2 |x| - 1 of the elements'
-// bits, so zeros (2^32 - 1) do not count; below kTinyCode some nonzero element
-// was under 2^-100.  It is taken from x itself and not from its first term,
-// which is zero for |x| <= 2^-134.
-constexpr uint32_t kTinyCode = 2u * (27u << 23);  // 2 * the bits of 2^-100
+// Of the elements a thread stages: the smallest nonzero one, as 2 |x| - 1 of
+// its bits (so zeros, 2^32 - 1, do not count), and the largest |x|.  Taken
+// from x itself: its first term is zero for |x| <= 2^-134.
+struct Range {
+  uint32_t lo = 0xffffffffu;
+  float hi = 0.f;
+  __device__ __forceinline__ void add(float x, float y) {
+    lo = min(lo, min(2u * __float_as_uint(x) - 1u, 2u * __float_as_uint(y) - 1u));
+    // one instruction for both (fmaxf would first quiet each of them)
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(hi) : "v"(x), "v"(y));
+  }
+};
+constexpr uint32_t kLossyCode = 2u * (17u << 23);  // 2 * the bits of 2^-110
 
+// Two elements adjacent in k, split: w[p] holds term p of both, the lower k
+// in the low half.
 __device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2));
 }
-__device__ __forceinline__ void split_pair(float x, float y, uint32_t (&w)[3], uint32_t& tiny) {
-  tiny = min(tiny, min(2u * __float_as_uint(x) - 1u, 2u * __float_as_uint(y) - 1u));
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t (&w)[3], Range& range) {
+  range.add(x, y);
   w[0] = pack_bf16(x, y);
   x -= __builtin_bit_cast(float, w[0] << 16);
   y -= __builtin_bit_cast(float, w[0] & 0xffff0000u);
@@ -98,17 +106,17 @@ struct Operand {
   __device__ __forceinline__ static int kof(int u) { return 4 * (u % 4); }
 
   // v: the unit's float4s, KC: v[j] = row j; !KC: v[e] = k e
-  __device__ __forceinline__ static void store(char* lds, int u, const f32x4 (&v)[4], uint32_t& tiny) {
+  __device__ __forceinline__ static void store(char* lds, int u, const f32x4 (&v)[4], Range& range) {
     char* p = lds + (u % 4 >> 1) * HS + (u & 1) * 8;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       uint32_t lo[3], hi[3];
       if (KC) {
-        split_pair(v[j][0], v[j][1], lo, tiny);
-        split_pair(v[j][2], v[j][3], hi, tiny);
+        split_pair(v[j][0], v[j][1], lo, range);
+        split_pair(v[j][2], v[j][3], hi, range);
       } else {
-        split_pair(v[0][j], v[1][j], lo, tiny);
-        split_pair(v[2][j], v[3][j], hi, tiny);
+        split_pair(v[0][j], v[1][j], lo, range);
+        split_pair(v[2][j], v[3][j], hi, range);
       }
 #pragma unroll
       for (int t = 0; t < 3; ++t) *reinterpret_cast<u32x2*>(p + t * PLANE + row(u, j) * 16) = u32x2{lo[t], hi[t]};
@@ -296,12 +304,13 @@ struct Tile {
   static constexpr int RED = C::WGK == 2 ? 4 * C::WM * C::WN * 16 * 64 * 4 : 0;  // reduce_wgk's bytes
   static constexpr int LDS = 2 * C::WGK * SB > RED ? 2 * C::WGK * SB : RED;
 
-  // Returns whether some staged element of the block was nonzero and below
-  // 2^-100; ends with a barrier.
+  // Adds to `range` what this thread stages; returns whether some element that
+  // the block has staged so far was nonzero and below 2^-110.  Ends with a
+  // barrier.
   template <bool EDGE>
   __device__ __forceinline__ static bool loop(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
                                              int64_t N, int64_t m0, int64_t n0, int64_t k_begin, int64_t k_end,
-                                             char* lds, bool neg, f32x16 (&acc)[C::WM][C::WN]) {
+                                             char* lds, bool neg, Range& range, f32x16 (&acc)[C::WM][C::WN]) {
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int grp = wave >> 2;                              // ping-pong group
     const int kg = C::WGK == 2 ? grp : 0;                   // k group
@@ -325,7 +334,6 @@ struct Tile {
     // load (256 x 256: 2.2 us), two in the short rounds of the smaller tiles
     // (128 x 128: 0.84 -> 0.73 us a round), one where two blocks share a CU
     f32x4 v0[4], v1[4];
-    uint32_t tiny = 0xffffffffu;
     auto load = [&](int t, f32x4 (&v)[4]) {
       if (!doA && !doB) return;
       if (!EDGE || t != tail) ld.load(v);
@@ -344,10 +352,10 @@ struct Tile {
         for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[j][e] = __uint_as_float(__float_as_uint(v[j][e]) ^ sign);
-        OA::store(b, ub, v, tiny);
+        OA::store(b, ub, v, range);
       } else {
         if (EDGE && t == tail) ld.place_tail<!TB>(kof, left, v);
-        OB::store(b + OA::BYTES, ub, v, tiny);
+        OB::store(b + OA::BYTES, ub, v, range);
       }
     };
     int wm, wn, wk;
@@ -397,31 +405,50 @@ struct Tile {
       if (t < nt) round(t, v1);
     }
     if (!grp) __syncthreads();
-    return __syncthreads_or(tiny < kTinyCode);
+    return __syncthreads_or(range.lo < kLossyCode);
   }
 
-  // neg (WGK == 1, no place to park): form the negated sum first.
-  __device__ __forceinline__ static bool run(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
+  // The block's largest staged |x|, for every thread; lds is free before and
+  // after.
+  __device__ __forceinline__ static float largest(char* lds, float hi) {
+    uint32_t* m = reinterpret_cast<uint32_t*>(lds);
+    if (threadIdx.x == 0) *m = 0;
+    __syncthreads();
+    atomicMax(m, __float_as_uint(hi));
+    __syncthreads();
+    hi = __uint_as_float(__builtin_amdgcn_readfirstlane(*m));
+    __syncthreads();
+    return hi;
+  }
+
+  // neg (WGK == 1, no place to park): form the negated sum first.  Returns the
+  // smallest output that the terms serve: 2^24 times what the block's operands
+  // may have lost in one (0 where they lost nothing).
+  __device__ __forceinline__ static float run(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
                                              int64_t N, int64_t m0, int64_t n0, int64_t k_begin, int64_t k_end,
                                              char* lds, const Park& park, bool neg, f32x16 (&acc)[C::WM][C::WN]) {
     const bool inside = m0 + C::BM <= M && n0 + C::BN <= N;
+    Range range;
+    auto floor = [&](bool lossy) {
+      return lossy ? largest(lds, range.hi) * ((float)(k_end - k_begin) * 0x1p-109f) : 0.f;
+    };
     auto part = [&](int64_t k0, int64_t k1, bool minus) {
-      return inside && (k1 - k0) % KT == 0 ? loop<false>(A, lda, B, ldb, M, N, m0, n0, k0, k1, lds, minus, acc)
-                                           : loop<true>(A, lda, B, ldb, M, N, m0, n0, k0, k1, lds, minus, acc);
+      return inside && (k1 - k0) % KT == 0 ? loop<false>(A, lda, B, ldb, M, N, m0, n0, k0, k1, lds, minus, range, acc)
+                                           : loop<true>(A, lda, B, ldb, M, N, m0, n0, k0, k1, lds, minus, range, acc);
     };
     if constexpr (C::WGK == 2) {
-      const bool any = part(k_begin, k_end, false);
+      const float least = floor(part(k_begin, k_end, false));
       if (threadIdx.x >= NS) negate<C>(acc);
       kp::reduce_wgk<C>(reinterpret_cast<float*>(lds), acc);
-      return any;
+      return least;
     }
     const int halves = park.C ? 2 : 1;
     const int64_t mid = park.C ? k_begin + (k_end - k_begin) / (2 * KT) * KT : k_end;
-    bool any = false, minus = neg;
+    bool lossy = false, minus = neg;
     int64_t k0 = k_begin, k1 = mid;
 #pragma unroll 1
     for (int half = 0;; ++half) {
-      any |= part(k0, k1, minus);
+      lossy = part(k0, k1, minus);
       if (half + 1 == halves) break;
       minus = true;
       k0 = mid;
@@ -442,7 +469,7 @@ struct Tile {
     }
     if (!park.C) {
       if (neg) negate<C>(acc);
-      return any;
+      return floor(lossy);
     }
     each_run<C>(acc, park, [&](f32x16& x, int e0, int64_t m, int64_t n) {
       if (n >= park.N) return;
@@ -457,87 +484,121 @@ struct Tile {
           if (m + e < park.M) x[e0 + e] = q[e] - x[e0 + e];
       }
     });
-    return any;
+    return floor(lossy);
   }
 
   // Whether this wave's outputs have to be formed with fp32 MFMAs: one is not
   // finite (an operand was not, or its bf16 term overflowed), or one is below
-  // 2^-60 while some operand element was below 2^-100, or one is nonzero and
-  // below 2^-84.
-  __device__ __forceinline__ static bool needs_fp32(const f32x16 (&acc)[C::WM][C::WN], bool tiny) {
-    float hi = 0.f, lo = INFINITY, lo_nz = INFINITY;
-    bool nan = false;
+  // `least` (run), zeros included.
+  __device__ __forceinline__ static bool needs_fp32(const f32x16 (&acc)[C::WM][C::WN], float least) {
+    float s[4] = {0.f, 0.f, 0.f, 0.f};  // NaN once a value was not finite
 #pragma unroll
     for (int i = 0; i < C::WM; ++i)
 #pragma unroll
       for (int j = 0; j < C::WN; ++j)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const float x = acc[i][j][e];
-          nan |= x != x;
-          hi = fmaxf(hi, fabsf(x));
-          lo = fminf(lo, fabsf(x));
-          lo_nz = fminf(lo_nz, x == 0.f ? INFINITY : fabsf(x));
-        }
-    const bool bad = nan || hi == INFINITY || (tiny && lo < 0x1p-60f) || lo_nz < 0x1p-84f;
-    return __any(bad);
+        for (int e = 0; e < 16; ++e) s[e & 3] = fmaf(acc[i][j][e], 0.f, s[e & 3]);
+    const float sum = (s[0] + s[1]) + (s[2] + s[3]);
+    if (least == 0.f) return __any(sum != sum);
+    float lo = INFINITY;
+#pragma unroll
+    for (int i = 0; i < C::WM; ++i)
+#pragma unroll
+      for (int j = 0; j < C::WN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) lo = fminf(lo, fabsf(acc[i][j][e]));
+    return __any(sum != sum || lo < least);
   }
 
-  // f(a, b): the wave's operand values at k, k + 1, straight from memory
-  // (zeros past the edges), over the whole contraction.
-  template <class F>
-  __device__ __forceinline__ static void each_k(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
-                                             int64_t N, int64_t m0, int64_t n0, int64_t k_begin, int64_t k_end, F&& f) {
-    int wm, wn, wk;
-    kp::wave_pos<C>(wm, wn, wk);
-    const int lane = threadIdx.x & 63, h = lane >> 5, r = lane & 31;
-    for (int64_t k = k_begin; k < k_end; k += 2) {
-      const int64_t kk = k + h;
-      float a[C::WM], b[C::WN];
+  // n >= 4 ? X(row, k .. k + 3) : those before k + n, then zeros; p at X(row, k)
+  template <bool KC, bool WHOLE>
+  __device__ __forceinline__ static f32x4 quad(const float* p, int64_t ld, int64_t n) {
+    f32x4 v;
+    if (KC && WHOLE) {
+      v = *reinterpret_cast<const f32x4u*>(p);
+    } else {
 #pragma unroll
-      for (int i = 0; i < C::WM; ++i) {
-        const int64_t m = m0 + wm * (C::WM * 32) + 32 * i + r;
-        a[i] = m < M && kk < k_end ? A[TA ? kk + lda * m : m + lda * kk] : 0.f;
-      }
-#pragma unroll
-      for (int j = 0; j < C::WN; ++j) {
-        const int64_t n = n0 + wn * (C::WN * 32) + 32 * j + r;
-        b[j] = n < N && kk < k_end ? B[!TB ? kk + ldb * n : n + ldb * kk] : 0.f;
-      }
-      f(a, b);
+      for (int e = 0; e < 4; ++e) v[e] = WHOLE || e < n ? p[KC ? e : ld * e] : 0.f;
     }
+    return v;
   }
 
-  // Whether this wave's operands hold a value of 2^30 or more: beside what a
-  // tiny value lost it can count in an output above 2^-60.
-  // Only asked where some element was below 2^-100; its code beside the loop
-  // and needs_fp32's test of small outputs cost the others up to 1.7%
-  // (1001 x 785 x 515 forward and backward 82.5 -> 83.9 us; 4096^3 nothing).
-  __device__ __forceinline__ static bool large(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
-                                            int64_t N, int64_t m0, int64_t n0, int64_t k_begin, int64_t k_end) {
-    float hi = 0.f;
-    each_k(A, lda, B, ldb, M, N, m0, n0, k_begin, k_end, [&](const float (&a)[C::WM], const float (&b)[C::WN]) {
-#pragma unroll
-      for (int i = 0; i < C::WM; ++i) hi = fmaxf(hi, fabsf(a[i]));
-#pragma unroll
-      for (int j = 0; j < C::WN; ++j) hi = fmaxf(hi, fabsf(b[j]));
-    });
-    return __any(hi >= 0x1p30f);
-  }
-
-  // The wave's outputs with v_mfma_f32_32x32x2f32: slow, for the rare waves
-  // that needs_fp32 or large names.
+  // The wave's outputs with v_mfma_f32_32x32x2f32, for the waves that
+  // needs_fp32 names; operands straight from memory, 8 k (4 per half-wave) a
+  // step and a stage of steps in flight behind the MFMAs, so the wave runs
+  // near the fp32 matrix rate.  Rows past the last are read from the last,
+  // their products never stored.
   __device__ __forceinline__ static void fp32(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
                                            int64_t N, int64_t m0, int64_t n0, int64_t k_begin, int64_t k_end,
                                            f32x16 (&acc)[C::WM][C::WN]) {
+    constexpr int D = C::WM * C::WN >= 8 ? 1 : C::WM * C::WN == 4 ? 2 : 4;  // steps of a stage
+    struct Stage {
+      f32x4 a[D][C::WM], b[D][C::WN];
+    };
+    int wm, wn, wk;
+    kp::wave_pos<C>(wm, wn, wk);
+    const int lane = threadIdx.x & 63, h = lane >> 5, r = lane & 31;
+    const float *pa[C::WM], *pb[C::WN];
+    const int64_t k0 = k_begin + 4 * h;
+#pragma unroll
+    for (int i = 0; i < C::WM; ++i) {
+      const int64_t m = min(m0 + wm * (C::WM * 32) + 32 * i + r, M - 1);
+      pa[i] = A + (TA ? k0 + lda * m : m + lda * k0);
+    }
+#pragma unroll
+    for (int j = 0; j < C::WN; ++j) {
+      const int64_t n = min(n0 + wn * (C::WN * 32) + 32 * j + r, N - 1);
+      pb[j] = B + (!TB ? k0 + ldb * n : n + ldb * k0);
+    }
+    const int64_t sa = TA ? 8 : 8 * lda, sb = !TB ? 8 : 8 * ldb;
+    auto step = [&](f32x4 (&a)[C::WM], f32x4 (&b)[C::WN], auto whole, int64_t left) {
+#pragma unroll
+      for (int i = 0; i < C::WM; ++i) {
+        a[i] = quad<TA, decltype(whole)::value>(pa[i], lda, left);
+        pa[i] += sa;
+      }
+#pragma unroll
+      for (int j = 0; j < C::WN; ++j) {
+        b[j] = quad<!TB, decltype(whole)::value>(pb[j], ldb, left);
+        pb[j] += sb;
+      }
+    };
+    auto load = [&](Stage& s) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) step(s.a[d], s.b[d], std::true_type{}, 4);
+    };
+    auto multiply = [&](const f32x4 (&a)[C::WM], const f32x4 (&b)[C::WN]) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < C::WM; ++i)
+#pragma unroll
+          for (int j = 0; j < C::WN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+    };
+    auto use = [&](const Stage& s) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) multiply(s.a[d], s.b[d]);
+    };
     kp::zero_acc<C>(acc);
-    each_k(A, lda, B, ldb, M, N, m0, n0, k_begin, k_end, [&](const float (&a)[C::WM], const float (&b)[C::WN]) {
-#pragma unroll
-      for (int i = 0; i < C::WM; ++i)
-#pragma unroll
-        for (int j = 0; j < C::WN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-    });
+    const int64_t stages = (k_end - k_begin) / (8 * D);
+    Stage s0, s1;
+    if (stages > 0) load(s0);
+    int64_t t = 0;
+#pragma unroll 1
+    for (; t + 1 < stages; t += 2) {
+      load(s1);
+      use(s0);
+      if (t + 2 < stages) load(s0);
+      use(s1);
+    }
+    if (t < stages) use(s0);
+#pragma unroll 1
+    for (int64_t k = k0 + stages * (8 * D); k - 4 * h < k_end; k += 8) {
+      f32x4 a[C::WM], b[C::WN];
+      step(a, b, std::false_type{}, k_end - k);
+      multiply(a, b);
+    }
   }
 };
 

@@ -161,6 +161,55 @@ def test_gemm_split_low_end_of_the_range(gpu, M, N, K, case, sign):
     assert bool((err <= lim).all()), f"worst error / bound {float((err / lim).max()):.3g}"
 
 
+def timed(fn):
+    """Milliseconds of one call, the best of 5 groups of 5."""
+    fn()
+    best = float("inf")
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(5):
+            fn()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) / 5)
+    return best
+
+
+@pytest.mark.parametrize("kind,limit", [("tails", 1.4), ("dead", 4.0), ("nan", 4.0)])
+@pytest.mark.parametrize("B,I,O", [(8192, 2048, 512), (4096, 4096, 4096)])
+def test_gemm_split_values_at_the_low_end_are_not_slow(gpu, B, I, O, kind, limit):
+    """Activations of which some lie below 2^-110 (GELU tails, the
+    probabilities of a peaked softmax) cost next to nothing beside ordinary
+    outputs; where every wave has to be formed again (an output that is zero
+    beside such a value, or a NaN in every column) the product costs the fp32
+    matrix rate on top, not memory's latency."""
+    gen = torch.Generator("cuda").manual_seed(B)
+    X = torch.randn(I, B, generator=gen, device="cuda")
+    W = torch.randn(O, I, generator=gen, device="cuda") / I ** 0.5
+    b = torch.zeros(O, device="cuda")
+    Y = torch.empty(O, B, device="cuda")
+    run = lambda: ops.linear_forward(X, W, b, Y, B, I, O)  # noqa: E731
+    plain = timed(run)
+    X[:, ::7] *= 2.0 ** -118 if kind != "nan" else 1.0
+    X[::3, 1::7] *= 2.0 ** -118 if kind != "nan" else 1.0
+    if kind == "tails":
+        X[:, ::7] *= 2.0 ** 118
+    if kind == "dead":
+        W[::16] = 0
+    if kind == "nan":
+        X[0, ::16] = float("nan")
+    slow = timed(run)
+    want = W.double() @ X.double()
+    ok = want.isfinite()
+    assert torch.equal(Y.isfinite(), ok)
+    size = (W.double().square() @ X.double().square()).sqrt()
+    lim = 8 * 2.0 ** -24 * (I / 2) ** 0.5 * size + I * 2.0 ** -149
+    assert bool(((Y.double() - want).abs()[ok] <= lim[ok]).all())
+    print(f"[split] {B}x{I}x{O} {kind}: {plain:.4f} -> {slow:.4f} ms", flush=True)
+    assert slow <= limit * plain, f"{plain:.4f} ms ordinary, {slow:.4f} ms with {kind}"
+
+
 def test_linear_residual_in_place(gpu):
     """The skip branch added into its own buffer (Z is Y): a tile whose half
     sums would wait in C must not clobber it."""
