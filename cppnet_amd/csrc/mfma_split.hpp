@@ -61,8 +61,9 @@ struct Range {
   uint32_t lo = 0xffffffffu;
   float hi = 0.f;
   __device__ __forceinline__ void add(float x, float y) {
-    lo = min(lo, min(2u * __float_as_uint(x) - 1u, 2u * __float_as_uint(y) - 1u));
-    // one instruction for both (fmaxf would first quiet each of them)
+    // one instruction each for both elements (the compiler regroups the minima
+    // of several pairs, and quiets the operands of fmaxf first)
+    asm("v_min3_u32 %0, %1, %2, %0" : "+v"(lo) : "v"(2u * __float_as_uint(x) - 1u), "v"(2u * __float_as_uint(y) - 1u));
     asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(hi) : "v"(x), "v"(y));
   }
 };
@@ -229,22 +230,33 @@ __device__ __forceinline__ void frags(const char* la, bf16x8 (&a)[C::WM][3], bf1
   }
 }
 
+// Whether a wave has the registers for a second accumulator, `low`, of the
+// five products that hold a remainder: they are 2^-8 of the result, so what
+// the matrix core cuts from their sum is too, and the leading products'
+// accumulator is cut once per k-tile and not six times (weight gradient of a
+// 1001 x 785 -> 515 layer against float64 1.55e-7 -> 1.29e-7; no time).  With
+// it the waves of 64 x 64 spill inside the k loop (8192 x 512 x 2048 103 ->
+// 181 us).
+template <class C>
+constexpr bool low_sums() { return C::WM * C::WN <= 2; }
+
 template <class C>
 __device__ __forceinline__ void mfmas(const bf16x8 (&a)[C::WM][3], const bf16x8 (&b)[C::WN][3],
-                                      f32x16 (&acc)[C::WM][C::WN]) {
-  auto term = [&](int x, int y) {
+                                      f32x16 (&acc)[C::WM][C::WN], f32x16 (&low)[C::WM][C::WN]) {
+  auto term = [&](int x, int y, f32x16 (&to)[C::WM][C::WN]) {
 #pragma unroll
     for (int i = 0; i < C::WM; ++i)
 #pragma unroll
       for (int j = 0; j < C::WN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][x], b[j][y], acc[i][j], 0, 0, 0);
+        to[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][x], b[j][y], to[i][j], 0, 0, 0);
   };
-  term(2, 0);
-  term(0, 2);
-  term(1, 1);
-  term(1, 0);
-  term(0, 1);
-  term(0, 0);
+  f32x16(&rest)[C::WM][C::WN] = low_sums<C>() ? low : acc;
+  term(2, 0, rest);
+  term(0, 2, rest);
+  term(1, 1, rest);
+  term(1, 0, rest);
+  term(0, 1, rest);
+  term(0, 0, acc);
 }
 
 template <class C>
@@ -364,6 +376,8 @@ struct Tile {
     const int ra = wm * (C::WM * 32) + r, rb = wn * (C::WN * 32) + r;
 
     constexpr int PF = C::WM * C::WN == 2 || C::WM * C::WN == 4 ? 2 : 1;
+    f32x16 low[C::WM][C::WN];
+    kp::zero_acc<C>(low);
     // one round: v holds k-tile t + 1
     auto round = [&](int t, f32x4 (&v)[4]) {
       bf16x8 a[C::WM][3], b[C::WN][3];
@@ -381,7 +395,7 @@ struct Tile {
       __builtin_amdgcn_sched_barrier(0);
       if (t < mine) {
         __builtin_amdgcn_s_setprio(1);
-        mfmas<C>(a, b, acc);
+        mfmas<C>(a, b, acc, low);
         __builtin_amdgcn_s_setprio(0);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -405,6 +419,12 @@ struct Tile {
       if (t < nt) round(t, v1);
     }
     if (!grp) __syncthreads();
+    if constexpr (low_sums<C>()) {
+#pragma unroll
+      for (int i = 0; i < C::WM; ++i)
+#pragma unroll
+        for (int j = 0; j < C::WN; ++j) acc[i][j] += low[i][j];
+    }
     return __syncthreads_or(range.lo < kLossyCode);
   }
 

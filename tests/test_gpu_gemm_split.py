@@ -161,6 +161,23 @@ def test_gemm_split_low_end_of_the_range(gpu, M, N, K, case, sign):
     assert bool((err <= lim).all()), f"worst error / bound {float((err / lim).max()):.3g}"
 
 
+# relative error measured with the fp32 MFMA tiles on these inputs:
+# what the split form must not exceed (with 3% for the plan's split counts)
+@pytest.mark.parametrize("B,I,O,fp32", [(1001, 785, 515, 1.435e-7), (292, 490, 2842, 1.142e-7), (3726, 224, 47, 1.444e-7)])
+def test_gemm_split_weight_gradient_error(gpu, B, I, O, fp32):
+    """X^T dY of a hidden layer (half of both operands zero), where an fp32
+    product of zero adds no rounding: the 2-norm error against float64 stays
+    within that of the fp32 MFMA."""
+    gen = torch.Generator("cuda").manual_seed(B)
+    r = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    X, dY = torch.relu(r(I, B)), torch.relu(r(O, B)) * r(O, B)
+    gW = torch.empty(O, I, device="cuda")
+    ops.gemm(True, False, I, O, B, X, B, dY, B, gW, I)
+    want = dY.double() @ X.double().T.contiguous()
+    err = float((gW.double() - want).norm() / want.norm())
+    assert err <= 1.03 * fp32, f"{err:.3e} against {fp32:.3e} of the fp32 MFMA"
+
+
 def timed(fn):
     """Milliseconds of one call, the best of 5 groups of 5."""
     fn()
