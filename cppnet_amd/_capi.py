@@ -51,6 +51,8 @@ SIGNATURES: dict[str, tuple] = {
                              i32, vp]),
     "cnhip_gemm_f32_batched": (i32, [i32, i32, i64, i64, i64, f32, vp, i64, i64, vp, i64, i64,
                                      f32, vp, i64, i64, i64, vp]),
+    "cnhip_gemm_f32_plan": (i32, [i32, i32, i64, i64, i64, i64, i64, i64, i32, C.POINTER(i32), C.POINTER(i32),
+                                  C.POINTER(i32), C.POINTER(i64), C.POINTER(C.c_size_t)]),
     "cnhip_gemm_timing_enable": (i32, [i32]),
     "cnhip_gemm_timing_read": (i32, [C.POINTER(i64), C.POINTER(C.c_double), C.POINTER(C.c_double)]),
     "cnhip_hbm_timing_enable": (i32, [i32]),

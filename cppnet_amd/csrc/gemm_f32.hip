@@ -676,15 +676,37 @@ int64_t shape_tiles(Shape shape, int64_t M, int64_t N) {
   return 0;
 }
 
+void shape_tile(Shape shape, int* m, int* n) {
+  auto set = [&](auto cfg) {
+    *m = decltype(cfg)::BM;
+    *n = decltype(cfg)::BN;
+  };
+  switch (shape) {
+    case Shape::XX: return set(CfgXX{});
+    case Shape::M: return set(CfgM{});
+    case Shape::N: return set(CfgN{});
+    case Shape::Q: return set(CfgQ{});
+    case Shape::SN: return set(CfgSN{});
+    case Shape::SM: return set(CfgSM{});
+    case Shape::S: return set(CfgS{});
+  }
+}
+
+// The k of one of `splits` splits, a multiple of KQ.
+int64_t k_per_split(int64_t K, int64_t splits) {
+  const int64_t k = (K + splits - 1) / splits;
+  return std::max((k + KQ - 1) / KQ * KQ, KQ);
+}
+
 // Cost of one launch: dispatch rounds times the k-tiles of one split, plus
 // the fixed-order reduce of split-K partials (read splits + 1 times M*N
-// floats, and a launch), over split counts min_s, 2 min_s, .. (INFINITY when
-// there is none).  A split count that leaves a nearly empty last round
+// floats, and a launch), over the split counts that the shape takes (INFINITY
+// when there is none).  A split count that leaves a nearly empty last round
 // costs a whole extra round, so it is avoided.  Splits keep >= 2 k-tiles of
 // 32 (4 for the fp32 shapes).  Returns the estimated seconds and the best
-// split count.
+// split count.  can_park: a 256 x 256 tile may keep a half sum in C.
 double split_cost(Shape shape, int64_t M, int64_t N, int64_t K, int64_t batches, int max_splits, int& splits,
-                  int64_t min_s = 1) {
+                  bool can_park = true) {
   const ShapeCost c = shape_cost(shape);
   const int64_t blocks = shape_tiles(shape, M, N) * batches;
   const bool fp32 = shape == Shape::SN || shape == Shape::SM || shape == Shape::S;
@@ -692,15 +714,20 @@ double split_cost(Shape shape, int64_t M, int64_t N, int64_t K, int64_t batches,
   if (blocks < c.slots && K >= 8 * KQ)
     max_s = std::max<int64_t>(1, std::min<int64_t>(K / ((fp32 ? 4 : 2) * KQ), max_splits));
   if (!fp32) max_s = std::max<int64_t>(1, std::min<int64_t>(max_s, kMaxPartialBytes / (M * N * batches * 4)));
-  if (max_s < min_s) return INFINITY;
-  double best = 0.0;
+  double best = INFINITY;
   splits = 1;
-  for (int64_t s = min_s; s <= max_s; s += min_s) {
+  for (int64_t s = 1; s <= max_s; ++s) {
+    // every contraction of a 256 x 256 tile is two half sums: parked in C, or
+    // as many positive splits as negated ones once k_per_split has rounded
+    if (shape == Shape::XX) {
+      const int64_t n = (K + k_per_split(K, s) - 1) / k_per_split(K, s);
+      if (n == 1 ? !can_park : n % 2 != 0) continue;
+    }
     const int64_t kt = ((K + s - 1) / s + KQ - 1) / KQ;
     const int64_t rounds = (blocks * s + c.slots - 1) / c.slots;
     double cost = (double)rounds * ((double)kt * c.t_tile + c.t_round);
     if (s > 1) cost += (double)(s + 1) * M * N * batches * 4.0 / 5e12 + 3e-6;
-    if (s == min_s || cost < best) {
+    if (cost < best) {
       best = cost;
       splits = (int)s;
     }
@@ -730,8 +757,7 @@ Plan plan_gemm(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_
     double best = 0.0;
     for (Shape c : {Shape::XX, Shape::M, Shape::N, Shape::Q}) {
       int sc = 1;
-      const bool whole = c != Shape::XX || (can_park && K >= kParkMinK);
-      const double cost = split_cost(c, M, N, K, batches, std::min(max_splits, 16), sc, whole ? 1 : 2);
+      const double cost = split_cost(c, M, N, K, batches, std::min(max_splits, 16), sc, can_park && K >= kParkMinK);
       if (c == Shape::XX || cost < best) {
         best = cost;
         shape = c;
@@ -739,9 +765,7 @@ Plan plan_gemm(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_
       }
     }
   }
-  int64_t kps = (K + splits - 1) / splits;
-  kps = ((kps + KQ - 1) / KQ) * KQ;
-  if (kps == 0) kps = KQ;
+  const int64_t kps = k_per_split(K, splits);
   splits = K > 0 ? (int)((K + kps - 1) / kps) : 1;
 
   return Plan{shape, shape_tiles(shape, M, N), splits, kps};
@@ -1146,6 +1170,26 @@ extern "C" int cnhip_gemm_f32_batched(int trans_a, int trans_b, int64_t M, int64
                                  stride_b, beta, C, ldc, stride_c, batch_count, nullptr,
                                  CNHIP_EPI_NONE, cnhip::as_stream(stream),
                                  "cnhip_gemm_f32_batched");
+}
+
+extern "C" int cnhip_gemm_f32_plan(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                   int64_t batch_count, int reads_c, int* tile_m, int* tile_n, int* splits,
+                                   int64_t* k_per_split, size_t* scratch_bytes) {
+  const char* who = "cnhip_gemm_f32_plan";
+  CNHIP_REQUIRE(M > 0 && N > 0 && K >= 0 && batch_count > 0, "%s: bad shape", who);
+  CNHIP_REQUIRE(tile_m && tile_n && splits && k_per_split && scratch_bytes, "%s: NULL argument", who);
+  using namespace cnhip;
+  *tile_m = *tile_n = 0;
+  *splits = 1;
+  *k_per_split = K;
+  *scratch_bytes = 0;
+  if (gemm_is_small(M, N, K, batch_count, trans_a, trans_b)) return CNHIP_OK;
+  const Plan p = plan_gemm(trans_a, trans_b, M, N, K, lda, ldb, batch_count, reads_c == 0, 64);
+  shape_tile(p.shape, tile_m, tile_n);
+  *splits = p.splits;
+  *k_per_split = p.kps;
+  *scratch_bytes = split_bytes(p, M, N, batch_count);
+  return CNHIP_OK;
 }
 
 extern "C" int cnhip_gemm_timing_enable(int on) {

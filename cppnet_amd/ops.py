@@ -9,6 +9,8 @@ non-zero status and refuse host tensors.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _capi
@@ -53,6 +55,15 @@ def gemm_batched(trans_a: bool, trans_b: bool, M: int, N: int, K: int, A, lda: i
                  beta: float = 0.0) -> None:
     _capi.call("cnhip_gemm_f32_batched", int(trans_a), int(trans_b), M, N, K, alpha, _p(A, "A"),
                lda, sa, _p(B, "B"), ldb, sb, beta, _p(C, "C"), ldc, sc, batch, _stream())
+
+
+def gemm_plan(trans_a: bool, trans_b: bool, M: int, N: int, K: int, lda: int, ldb: int, batch: int = 1,
+              reads_c: bool = False) -> tuple[int, int, int, int, int]:
+    """(tile rows, tile columns, splits, k per split, scratch bytes) of a product; no GPU needed."""
+    m, n, s, k, b = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_int64(), ctypes.c_size_t()
+    _capi.call("cnhip_gemm_f32_plan", int(trans_a), int(trans_b), M, N, K, lda, ldb, batch, int(reads_c), ctypes.byref(m),
+               ctypes.byref(n), ctypes.byref(s), ctypes.byref(k), ctypes.byref(b))
+    return m.value, n.value, s.value, k.value, b.value
 
 
 def linear_forward(X, W, b, Y, batch: int, in_features: int, out_features: int) -> None:

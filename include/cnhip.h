@@ -124,6 +124,13 @@ int cnhip_gemm_f32_batched(int trans_a, int trans_b, int64_t M, int64_t N, int64
                            float* C, int64_t ldc, int64_t stride_c, int64_t batch_count,
                            cnhip_stream_t stream);
 
+/* How the two functions above would run a product (no GPU is needed): the
+ * output tile of a block (0 x 0: one of the kernels for tiny products), the
+ * splits of K, the k of each, and the bytes of their partial sums.  reads_c:
+ * beta != 0.  Not a reference function. */
+int cnhip_gemm_f32_plan(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                        int64_t batch_count, int reads_c, int* tile_m, int* tile_n, int* splits,
+                        int64_t* k_per_split, size_t* scratch_bytes);
 
 /* Measurement aid for the MFMA GEMM-shaped kernels (the GEMM kernel and the
  * implicit-GEMM Conv2D forward / dgrad / wgrad kernels): while enabled,

@@ -1,0 +1,48 @@
+"""How the GEMM splits its work, over random sizes (the planner runs on the
+host and needs no GPU)."""
+import math
+import random
+
+import pytest
+
+from cppnet_amd import ops
+
+
+def sizes(n, seed):
+    rng = random.Random(seed)
+    for _ in range(n):
+        M, N, K = (int(round(math.exp(rng.uniform(math.log(33), math.log(12000))))) for _ in range(3))
+        yield M, N, K, rng.choice([1, 1, 1, 1, rng.randint(2, 300)]), rng.random() < 0.5, rng.random() < 0.5
+
+
+def plan(M, N, K, batch=1, ta=False, tb=False, reads_c=False):
+    return ops.gemm_plan(ta, tb, M, N, K, K if ta else M, N if tb else K, batch, reads_c)
+
+
+def check_halves(tile, splits, reads_c):
+    # a 256 x 256 tile forms two half sums of opposite sign: one after the
+    # other in C, or in an even number of splits
+    if tile == (256, 256):
+        assert splits % 2 == 0 or (splits == 1 and not reads_c), splits
+
+
+@pytest.mark.parametrize("M,N,K", [(162, 6975, 9148), (5559, 136, 9583), (143, 3229, 6674), (4096, 4096, 4096), (300, 500, 400)])
+@pytest.mark.parametrize("reads_c", [False, True])
+def test_large_tiles_run_as_two_half_sums(M, N, K, reads_c):
+    m, n, splits, _, _ = plan(M, N, K, reads_c=reads_c)
+    check_halves((m, n), splits, reads_c)
+
+
+def test_plans_cover_the_product():
+    for M, N, K, batch, ta, tb in sizes(3000, 5):
+        for reads_c in (False, True):
+            m, n, splits, kps, scratch = plan(M, N, K, batch, ta, tb, reads_c)
+            what = (M, N, K, batch, ta, tb, reads_c, m, n, splits, kps)
+            if m == 0:
+                continue
+            check_halves((m, n), splits, reads_c)
+            # every split has work, and all of them together cover K
+            assert kps % 32 == 0 and (splits - 1) * kps < K <= splits * kps, what
+            assert scratch == (splits * M * N * batch * 4 if splits > 1 else 0), what
+            # the partial sums stay within the no-allocation entry points' array
+            assert scratch <= 32 << 20, what
