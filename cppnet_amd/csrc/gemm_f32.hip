@@ -6,22 +6,23 @@
 // (forward NN, weight-grad TN, input-grad NT; ref: matmul.cu:16-71,
 // matmul_grad_weight.cu:14-69, matmul_grad_input.cu:14-68) and the batched
 // products of the recurrent and attention layers.  The reference computes one
-// output per thread with atomicAdd accumulation.  Here a block of 8 wave64s
-// owns an output tile of up to 256 x 256 and forms it on the bf16 matrix
-// cores from operands split into three bf16 terms (mfma_split.hpp), with the
-// error of an fp32 sum; skinny products use fp32 MFMA tiles
-// (mfma_kpack.hpp), tiny ones plain FMAs; no atomics are used.  When the
-// output tiles alone cannot fill the 256 CUs, K is split across blocks into
-// a stream-ordered workspace and the partials are summed in a fixed order,
-// so results are deterministic.
+// output per thread with atomicAdd accumulation.  Here large products run on
+// the bf16 matrix cores from operands split into three bf16 terms, with the
+// error of an fp32 sum: a block of 8 wave64s owns a tile of 256 x 256 or
+// 128 x 128 (mfma_split.hpp).  All others run on fp32 MFMAs in 64 x 64 or
+// skinny tiles (mfma_kpack.hpp), tiny ones on plain FMAs; no atomics are used.
+// When the output tiles alone cannot fill the 256 CUs, K is split across
+// blocks into a stream-ordered workspace and the partials are summed in a
+// fixed order, so results are deterministic.
 //
-// Measured on MI355X, fp32 MFMA tiles before -> split operands: 4096^3 980 ->
-// 625-640 us (219 TFLOP/s; the bf16 pipe alone would take 453 us at the
-// 1.82 PFLOP/s that the card's power limit leaves it), 8192 x 512 x 2048 144
-// -> 95 us, 8192 x 2048 x 512 160 -> 112 us, 32 x (256 x 512 x 256) 25 -> 21 us.
+// Measured on MI355X, fp32 MFMA tiles -> split operands: 4096^3 980 ->
+// 625-640 us (219 TFLOP/s; the bf16 pipe alone would take 461 us at the
+// 1.79 PFLOP/s that the card's power limit leaves it on random operands),
+// 8192 x 512 x 2048 144 -> 95 us, 8192 x 2048 x 512 160 -> 112 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <cstring>
 #include <vector>
 
@@ -38,17 +39,14 @@ using kp::f32x16;
 using kp::f32x4;
 using sp::f32x4u;
 
-// Tile shapes.  The products of large and medium shape run on the bf16 matrix
-// cores with their operands split in three (mfma_split.hpp), 8 waves a block;
-// the fp32 MFMA keeps the skinny ones, and operands whose rows lie so far
-// apart that 32-bit offsets do not span a tile.
-using CfgXX = kp::Cfg<2, 4, 4, 2>;           // 256 x 256, waves of 128x64, k whole
-using CfgM = kp::Cfg<2, 2, 2, 2, 16, 2>;     // 128 x 128, 2 k groups of 4 waves of 64x64
-using CfgN = kp::Cfg<2, 2, 2, 1, 16, 2>;     // 128 x 64, 2 k groups of 4 waves of 64x32
-using CfgQ = kp::Cfg<2, 2, 1, 1, 16, 2>;     // 64 x 64, 2 k groups of 4 waves of 32x32
-using CfgSN = kp::Cfg<4, 1, 1, 1>;           // 128 x 32 : N <= 32, fp32 MFMA
-using CfgSM = kp::Cfg<1, 4, 1, 1>;           // 32 x 128 : M <= 32, fp32 MFMA
-using CfgS = kp::Cfg<2, 2, 1, 1>;            // 64 x 64, fp32 MFMA: any leading dimension
+// Tile shapes.  Large products of even sizes run on the bf16 matrix cores with
+// their operands split in three (mfma_split.hpp), 8 waves a block; the fp32
+// MFMA takes all others (plan_gemm).
+using CfgXX = kp::Cfg<2, 4, 4, 2>;           // 256 x 256, waves of 128x64, k whole; split operands
+using CfgM = kp::Cfg<2, 2, 2, 2, 16, 2>;     // 128 x 128, 2 k groups of 4 waves of 64x64; split operands
+using CfgSN = kp::Cfg<4, 1, 1, 1>;           // 128 x 32 : N <= 32
+using CfgSM = kp::Cfg<1, 4, 1, 1>;           // 32 x 128 : M <= 32
+using CfgS = kp::Cfg<2, 2, 1, 1>;            // 64 x 64, summed in two levels (kp::BlockSums)
 
 template <class C>
 constexpr bool split_cfg() { return C::NT == 512; }
@@ -57,9 +55,9 @@ constexpr bool split_cfg() { return C::NT == 512; }
 constexpr int64_t KQ = 32;
 
 // Waves per SIMD to leave registers for: the split shapes run one 8-wave
-// block per CU, the smallest of them two; the 4-wave fp32 shapes two.
-template <class C>
-constexpr int min_waves() { return split_cfg<C>() && C::BM * C::BN <= 64 * 64 ? 4 : 2; }
+// block per CU; the 64 x 64 tile, left alone, takes 96 or 106 registers (four
+// blocks a CU).
+constexpr int kMinWaves = 2;
 
 struct GemmArgs {
   int64_t M, N, K;
@@ -177,7 +175,19 @@ __device__ __forceinline__ void gemm_mainloop(const GemmArgs& g, const float* __
                                               f32x16 (&acc)[C::WM][C::WN]) {
   const int ntiles = k_end > k_begin ? (int)((k_end - k_begin + C::BK - 1) / C::BK) : 0;
   GemmStage<FAST, TA, TB, C> s(g, A, B, m0, n0, k_begin, k_end);
-  kp::pipeline<C>(ntiles, lds, s, acc);
+  if constexpr (std::is_same<C, CfgS>::value) {
+    kp::BlockSums<C> sums;
+    kp::zero_acc<C>(sums.four);
+    kp::zero_acc<C>(sums.total);
+    kp::pipeline<C>(ntiles, lds, s, sums);
+    kp::fold(sums);
+#pragma unroll
+    for (int i = 0; i < C::WM; ++i)
+#pragma unroll
+      for (int j = 0; j < C::WN; ++j) acc[i][j] = sums.total[i][j];
+  } else {
+    kp::pipeline<C>(ntiles, lds, s, acc);
+  }
 }
 
 // Accumulator block b (row-major over WM x WN) by a wave-uniform index.
@@ -372,7 +382,7 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& g, float* lds, int bx
 }
 
 template <bool TA, bool TB, class C, bool FUSED>
-__global__ void __launch_bounds__(C::NT, min_waves<C>()) gemm_f32_kernel(GemmArgs g) {
+__global__ void __launch_bounds__(C::NT, kMinWaves) gemm_f32_kernel(GemmArgs g) {
   __shared__ __align__(16) float lds[gemm_lds_floats<TA, TB, C>()];
   gemm_block<TA, TB, C, FUSED>(g, lds, (int)blockIdx.x, (int64_t)blockIdx.y, (int)blockIdx.z);
 }
@@ -382,7 +392,7 @@ __global__ void __launch_bounds__(C::NT, min_waves<C>()) gemm_f32_kernel(GemmArg
 // second's, each block exactly as in its own launch (so each product is
 // bit-identical to a launch of its own with the same plan).
 template <bool TA1, bool TB1, bool F1, bool TA2, bool TB2, bool F2, class C>
-__global__ void __launch_bounds__(C::NT, min_waves<C>()) gemm_pair_kernel(GemmArgs g1, GemmArgs g2, int n1,
+__global__ void __launch_bounds__(C::NT, kMinWaves) gemm_pair_kernel(GemmArgs g1, GemmArgs g2, int n1,
                                                                            int tiles1, int batches1, int tiles2,
                                                                            int batches2) {
   constexpr int F = gemm_lds_floats<TA1, TB1, C>() > gemm_lds_floats<TA2, TB2, C>()
@@ -622,7 +632,7 @@ TimingRec* hbm_timing_slot(const char* kernel, double bytes) {
 
 namespace {
 
-enum class Shape { XX, M, N, Q, SN, SM, S };
+enum class Shape { XX, M, SN, SM, S };
 
 template <class Cfg>
 int64_t tiles_of(int64_t M, int64_t N) {
@@ -640,35 +650,41 @@ struct Plan {
 // workspace of the no-allocation entry points, which run the same plans).
 constexpr int64_t kMaxPartialBytes = (int64_t)32 << 20;
 
-// What a tile shape costs: block slots of the chip, seconds per 32 of k of
-// one round of those slots, and seconds a round spends outside its k loop
-// (first loads, stores).  Fitted to sweeps of every shape and split count
-// over 28 sizes (from 4096 x 64 x 64 to 4096^3, all orientations): the plan
-// is within 5% of the best of them but for 1001 x 785 x 515 (8%).
+// What a tile shape costs: block slots of the chip; for each round of those
+// slots the seconds outside the k loop (first loads, stores) and, per 32 of k,
+// the latency of a block; per 32 of k and block of a CU the time its matrix
+// pipes need.  Fitted to sweeps of every shape and split count over 113 sizes
+// in the three orientations of a layer (64^3 to 4096^3 and 8192 x 2048 x 512,
+// ragged ones, batches up to 512, contractions up to 60000): the plan takes
+// 0.9% longer than the best of them in the mean, 30% at worst (2000^3, where
+// 256 x 256 tiles in two splits beat their edges' cost).
 struct ShapeCost {
   int64_t slots;
-  double t_tile, t_round;
+  double t_round, t_lat, t_tile;
 };
 
 ShapeCost shape_cost(Shape shape) {
   switch (shape) {
-    case Shape::XX: return {256, 4.5e-6, 10e-6};
-    case Shape::M: return {256, 1.42e-6, 6e-6};
-    case Shape::N: return {256, 1.05e-6, 5e-6};
-    case Shape::Q: return {512, 1.34e-6, 4e-6};
-    case Shape::SN: return {1024, 2.0 * CfgSN::BM * CfgSN::BN * KQ / (157.3e12 / 256) * 4 / 0.8, 0};
-    case Shape::SM: return {1024, 2.0 * CfgSM::BM * CfgSM::BN * KQ / (157.3e12 / 256) * 4 / 0.8, 0};
-    case Shape::S: return {1024, 2.0 * CfgS::BM * CfgS::BN * KQ / (157.3e12 / 256) * 4 / 0.8, 0};
+    case Shape::XX: return {256, 10.6e-6, 0, 3.53e-6};
+    case Shape::M: return {256, 5.31e-6, 0, 1.42e-6};
+    case Shape::S: return {1024, 2.0e-6, 1.31e-6, 0.501e-6};
+    case Shape::SN: return {1024, 0, 2.0 * CfgSN::BM * CfgSN::BN * KQ / (157.3e12 / 256) * 4 / 0.8, 0};
+    case Shape::SM: return {1024, 0, 2.0 * CfgSM::BM * CfgSM::BN * KQ / (157.3e12 / 256) * 4 / 0.8, 0};
   }
-  return {1024, 1e-6, 0};
+  return {1024, 0, 1e-6, 0};
 }
+
+// A block that has an edge or a last k-tile cut short checks (the split shapes
+// also place) what it stages in every k-tile, and as all blocks of a round wait
+// for it the whole product takes longer: by kSplitEdge and kEdge, and for the
+// split shapes kSplitTail more where K is no multiple of the k-tile (8102 x
+// 613 x 4079: 610 us, the 64 x 64 tile 395).
+constexpr double kSplitEdge = 1.45, kSplitTail = 1.06, kEdge = 1.21;
 
 int64_t shape_tiles(Shape shape, int64_t M, int64_t N) {
   switch (shape) {
     case Shape::XX: return tiles_of<CfgXX>(M, N);
     case Shape::M: return tiles_of<CfgM>(M, N);
-    case Shape::N: return tiles_of<CfgN>(M, N);
-    case Shape::Q: return tiles_of<CfgQ>(M, N);
     case Shape::SN: return tiles_of<CfgSN>(M, N);
     case Shape::SM: return tiles_of<CfgSM>(M, N);
     case Shape::S: return tiles_of<CfgS>(M, N);
@@ -684,8 +700,6 @@ void shape_tile(Shape shape, int* m, int* n) {
   switch (shape) {
     case Shape::XX: return set(CfgXX{});
     case Shape::M: return set(CfgM{});
-    case Shape::N: return set(CfgN{});
-    case Shape::Q: return set(CfgQ{});
     case Shape::SN: return set(CfgSN{});
     case Shape::SM: return set(CfgSM{});
     case Shape::S: return set(CfgS{});
@@ -698,35 +712,41 @@ int64_t k_per_split(int64_t K, int64_t splits) {
   return std::max((k + KQ - 1) / KQ * KQ, KQ);
 }
 
-// Cost of one launch: dispatch rounds times the k-tiles of one split, plus
-// the fixed-order reduce of split-K partials (read splits + 1 times M*N
-// floats, and a launch), over the split counts that the shape takes (INFINITY
-// when there is none).  A split count that leaves a nearly empty last round
-// costs a whole extra round, so it is avoided.  Splits keep >= 2 k-tiles of
-// 32 (4 for the fp32 shapes).  Returns the estimated seconds and the best
-// split count.  can_park: a 256 x 256 tile may keep a half sum in C.
+// Cost of one launch: its rounds and k-tiles (ShapeCost), plus the fixed-order
+// reduce of split-K partials (read splits + 1 times M*N floats, and a launch),
+// over the split counts that the shape takes (INFINITY when there is none).
+// A split count that leaves a nearly empty last round costs a whole extra
+// round, so it is avoided.  Splits keep >= 2 k-tiles of 32 (4 for the skinny
+// shapes).  Returns the estimated seconds and the best split count.
+// can_park: a 256 x 256 tile may keep a half sum in C.
 double split_cost(Shape shape, int64_t M, int64_t N, int64_t K, int64_t batches, int max_splits, int& splits,
                   bool can_park = true) {
   const ShapeCost c = shape_cost(shape);
   const int64_t blocks = shape_tiles(shape, M, N) * batches;
-  const bool fp32 = shape == Shape::SN || shape == Shape::SM || shape == Shape::S;
+  const bool skinny = shape == Shape::SN || shape == Shape::SM;
   int64_t max_s = 1;
   if (blocks < c.slots && K >= 8 * KQ)
-    max_s = std::max<int64_t>(1, std::min<int64_t>(K / ((fp32 ? 4 : 2) * KQ), max_splits));
-  if (!fp32) max_s = std::max<int64_t>(1, std::min<int64_t>(max_s, kMaxPartialBytes / (M * N * batches * 4)));
+    max_s = std::max<int64_t>(1, std::min<int64_t>(K / ((skinny ? 4 : 2) * KQ), max_splits));
+  if (!skinny) max_s = std::max<int64_t>(1, std::min<int64_t>(max_s, kMaxPartialBytes / (M * N * batches * 4)));
+  int tm = 0, tn = 0;
+  shape_tile(shape, &tm, &tn);
+  const bool split = shape == Shape::XX || shape == Shape::M;
+  double t_tile = c.t_tile;
+  if (!skinny && (M % tm != 0 || N % tn != 0 || K % sp::KT != 0)) t_tile *= split ? kSplitEdge : kEdge;
+  if (split && K % sp::KT != 0) t_tile *= kSplitTail;
   double best = INFINITY;
   splits = 1;
   for (int64_t s = 1; s <= max_s; ++s) {
+    const int64_t kps = k_per_split(K, s);
     // every contraction of a 256 x 256 tile is two half sums: parked in C, or
     // as many positive splits as negated ones once k_per_split has rounded
     if (shape == Shape::XX) {
-      const int64_t n = (K + k_per_split(K, s) - 1) / k_per_split(K, s);
+      const int64_t n = (K + kps - 1) / kps;
       if (n == 1 ? !can_park : n % 2 != 0) continue;
     }
-    const int64_t kt = ((K + s - 1) / s + KQ - 1) / KQ;
-    const int64_t rounds = (blocks * s + c.slots - 1) / c.slots;
-    double cost = (double)rounds * ((double)kt * c.t_tile + c.t_round);
-    if (s > 1) cost += (double)(s + 1) * M * N * batches * 4.0 / 5e12 + 3e-6;
+    const double kt = (double)(kps / KQ), rounds = (double)((blocks * s + c.slots - 1) / c.slots);
+    double cost = rounds * c.t_round + kt * std::max(rounds * c.t_lat, (double)((blocks * s + 255) / 256) * t_tile);
+    if (s > 1) cost += (double)(s + 1) * M * N * batches * 4.0 / 5.2e12 + 3.2e-6;
     if (cost < best) {
       best = cost;
       splits = (int)s;
@@ -740,25 +760,28 @@ double split_cost(Shape shape, int64_t M, int64_t N, int64_t K, int64_t batches,
 // 4096 x 4096 x 1024 at 201 us against 196, x 4096 at 638 against 716.
 constexpr int64_t kParkMinK = 1536;
 
-// A 256 x 256 tile without a half sum in C takes an even number of splits.
 // can_park: C is neither read (beta) nor the memory of the side tensor.
-Plan plan_gemm(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t batches,
-               bool can_park, int max_splits) {
-  // Skinny shapes take the 32-wide fp32 tiles (no MFMA work on padding), the
-  // rest the split shape and split count of the lowest cost.
+Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batches, bool offsets_fit, bool can_park, int max_splits) {
+  // Skinny shapes take the 32-wide tiles (no MFMA work on padding), the rest
+  // the shape and split count of the lowest cost.  The split shapes' 8-wave
+  // blocks hide neither their first loads nor their stores behind another
+  // block, so the 64 x 64 tile, four of whose blocks share a CU, is the faster
+  // one of all but large products of whole tiles: 128^3 5.8 us against 8.6 of
+  // the best split tile, 1024^3 23 against 27, 256 x (256 x 256 x 64) 31
+  // against 46, 1001 x 515 x 785 21 against 26; 2048 x 2048 x 512 40 against
+  // 32, 8192 x 512 x 2048 142 against 96, 4096^3 1130 against 630.
   Shape shape = Shape::S;
   int splits = 1;
   if (N <= 32 || M <= 32) {
     shape = N <= 32 ? Shape::SN : Shape::SM;
     split_cost(shape, M, N, K, batches, max_splits, splits);
-  } else if (K < sp::KT || !sp::offsets_fit(lda, trans_a != 0, CfgXX::BM) || !sp::offsets_fit(ldb, trans_b == 0, CfgXX::BN)) {
-    split_cost(shape, M, N, K, batches, max_splits, splits);
   } else {
-    double best = 0.0;
-    for (Shape c : {Shape::XX, Shape::M, Shape::N, Shape::Q}) {
+    double best = split_cost(Shape::S, M, N, K, batches, max_splits, splits);
+    for (Shape c : {Shape::XX, Shape::M}) {
+      if (K < sp::KT || !offsets_fit) break;
       int sc = 1;
       const double cost = split_cost(c, M, N, K, batches, std::min(max_splits, 16), sc, can_park && K >= kParkMinK);
-      if (c == Shape::XX || cost < best) {
+      if (cost < best) {
         best = cost;
         shape = c;
         splits = sc;
@@ -771,6 +794,26 @@ Plan plan_gemm(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_
   return Plan{shape, shape_tiles(shape, M, N), splits, kps};
 }
 
+// make_plan, a function of sizes alone, remembered for the sizes that a thread
+// uses: it tries about 100 split counts (2 us), as long as a short launch.
+Plan plan_gemm(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t batches,
+               bool can_park, int max_splits) {
+  struct Entry {
+    int64_t M, N, K, batches;
+    int how;
+    Plan plan;
+  };
+  static thread_local Entry memo[64] = {};
+  const bool fit = sp::offsets_fit(lda, trans_a != 0, CfgXX::BM) && sp::offsets_fit(ldb, trans_b == 0, CfgXX::BN);
+  const int how = max_splits << 2 | (fit ? 2 : 0) | (can_park ? 1 : 0);
+  const uint64_t h = ((uint64_t)M * 0x9E3779B97F4A7C15u ^ (uint64_t)N * 0xC2B2AE3D27D4EB4Fu ^
+                      (uint64_t)K * 0x165667B19E3779F9u ^ (uint64_t)batches * 0x27D4EB2F165667C5u) >> 58;
+  Entry& e = memo[h ^ (can_park ? 1 : 0)];
+  if (e.M != M || e.N != N || e.K != K || e.batches != batches || e.how != how)
+    e = Entry{M, N, K, batches, how, make_plan(M, N, K, batches, fit, can_park, max_splits)};
+  return e.plan;
+}
+
 // Launches the planned kernel, bracketed by the per-launch timing events.
 int launch_plan(Shape shape, int trans_a, int trans_b, const GemmArgs& g, int64_t batches,
                 hipStream_t st, const char* who) {
@@ -780,8 +823,6 @@ int launch_plan(Shape shape, int trans_a, int trans_b, const GemmArgs& g, int64_
   switch (shape) {
     case Shape::XX: launch_t<CfgXX>(trans_a, trans_b, g, batches, st); break;
     case Shape::M: launch_t<CfgM>(trans_a, trans_b, g, batches, st); break;
-    case Shape::N: launch_t<CfgN>(trans_a, trans_b, g, batches, st); break;
-    case Shape::Q: launch_t<CfgQ>(trans_a, trans_b, g, batches, st); break;
     case Shape::SN: launch_t<CfgSN>(trans_a, trans_b, g, batches, st); break;
     case Shape::SM: launch_t<CfgSM>(trans_a, trans_b, g, batches, st); break;
     case Shape::S: launch_t<CfgS>(trans_a, trans_b, g, batches, st); break;

@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace cnhip {
 namespace kp {
@@ -359,25 +360,54 @@ constexpr int stage_floats() {
   return Stage::OA::FLOATS + Stage::OB::FLOATS;
 }
 
-// Software pipeline over ntiles k-tiles: tile t+1 and t+2 are in flight in
-// two register sets while tile t is multiplied from LDS (double-buffered, one
-// barrier per k-tile).  The stage names its operands OA and OB and supplies
-// load<S>(t) (global -> register set S) and store<S>(buf) (register set S ->
-// an LDS buffer: A tile, then B tile at OA::FLOATS); the loop is unrolled by
-// two so the sets alternate statically.  lds holds 2 * stage_floats<Stage>().
-// The loop body runs whole tile pairs and has no exit in its middle, and an
-// odd last tile is done after it: with a single exit the accumulators keep
-// one register assignment around the loop (a mid-body exit made the compiler
-// copy every accumulator between two register sets each iteration).
-// Ends with a barrier, after which lds may be reused.
+// Accumulators in two levels: a k-tile's products are summed from zero, added
+// to the sum of 4 k-tiles, and that to the total.  A long contraction's
+// rounding error is then that of short sums and not of the whole length, for
+// 20 vector additions a k-tile of 8 MFMAs and up, which run beside them.
+template <class C>
+struct BlockSums {
+  f32x16 four[C::WM][C::WN], total[C::WM][C::WN];
+};
+template <class C>
+__device__ __forceinline__ void fold(BlockSums<C>& s) {
+#pragma unroll
+  for (int i = 0; i < C::WM; ++i)
+#pragma unroll
+    for (int j = 0; j < C::WN; ++j) s.total[i][j] += s.four[i][j];
+  zero_acc<C>(s.four);
+}
+
 template <class C, class OA, class OB, class Acc>
 __device__ __forceinline__ void ktile_any(const float* la, const float* lb, Acc& acc) {
-  if constexpr (sizeof(acc[0][0]) == sizeof(f32x16))
+  if constexpr (std::is_same<Acc, BlockSums<C>>::value) {
+    f32x16 part[C::WM][C::WN];
+    zero_acc<C>(part);
+    mfma_ktile<C, OA, OB>(la, lb, part);
+#pragma unroll
+    for (int i = 0; i < C::WM; ++i)
+#pragma unroll
+      for (int j = 0; j < C::WN; ++j) {
+        acc.four[i][j] += part[i][j];
+        asm volatile("" : "+v"(acc.four[i][j]));  // now: else four k-tiles' parts stay in registers
+      }
+  } else if constexpr (sizeof(acc[0][0]) == sizeof(f32x16))
     mfma_ktile<C, OA, OB>(la, lb, acc);
   else
     mfma_ktile16<C, OA, OB>(la, lb, acc);
 }
 
+// Software pipeline over ntiles k-tiles: tile t+1 and t+2 are in flight in
+// two register sets while tile t is multiplied from LDS (double-buffered, one
+// barrier per k-tile).  The stage names its operands OA and OB and supplies
+// load<S>(t) (global -> register set S) and store<S>(buf) (register set S ->
+// an LDS buffer: A tile, then B tile at OA::FLOATS); the loop is unrolled by
+// two so the sets alternate statically (by four with BlockSums, which are
+// folded there).  lds holds 2 * stage_floats<Stage>().
+// The loop body runs whole tile pairs and has no exit in its middle, and an
+// odd last tile is done after it: with a single exit the accumulators keep
+// one register assignment around the loop (a mid-body exit made the compiler
+// copy every accumulator between two register sets each iteration).
+// Ends with a barrier, after which lds may be reused.
 template <class C, class Stage, class Acc>
 __device__ __forceinline__ void pipeline(int ntiles, float* lds, Stage& s, Acc& acc) {
   using OA = typename Stage::OA;
@@ -393,19 +423,43 @@ __device__ __forceinline__ void pipeline(int ntiles, float* lds, Stage& s, Acc& 
   if (ntiles > 2) s.template load<1>(2);
   __syncthreads();
   int kt = 0;
-  for (; kt + 1 < ntiles; kt += 2) {
-    // tile kt in buf0, kt+1 in set 0, kt+2 in set 1
-    ktile_any<C, OA, OB>(buf0, buf0 + BOFF, acc);
-    s.template store<0>(buf1);
-    if (kt + 3 < ntiles) s.template load<0>(kt + 3);
-    __syncthreads();
-    // tile kt+1 in buf1, kt+2 in set 1, kt+3 in set 0
-    ktile_any<C, OA, OB>(buf1, buf1 + BOFF, acc);
-    if (kt + 2 < ntiles) {
-      s.template store<1>(buf0);
-      if (kt + 4 < ntiles) s.template load<1>(kt + 4);
+  if constexpr (std::is_same<Acc, BlockSums<C>>::value) {
+    auto pair = [&](int t) {  // as the loop body below
+      ktile_any<C, OA, OB>(buf0, buf0 + BOFF, acc);
+      s.template store<0>(buf1);
+      if (t + 3 < ntiles) s.template load<0>(t + 3);
+      __syncthreads();
+      ktile_any<C, OA, OB>(buf1, buf1 + BOFF, acc);
+      if (t + 2 < ntiles) {
+        s.template store<1>(buf0);
+        if (t + 4 < ntiles) s.template load<1>(t + 4);
+      }
+      __syncthreads();
+    };
+    for (; kt + 3 < ntiles; kt += 4) {
+      pair(kt);
+      pair(kt + 2);
+      fold(acc);
     }
-    __syncthreads();
+    if (kt + 1 < ntiles) {
+      pair(kt);
+      kt += 2;
+    }
+  } else {
+    for (; kt + 1 < ntiles; kt += 2) {
+      // tile kt in buf0, kt+1 in set 0, kt+2 in set 1
+      ktile_any<C, OA, OB>(buf0, buf0 + BOFF, acc);
+      s.template store<0>(buf1);
+      if (kt + 3 < ntiles) s.template load<0>(kt + 3);
+      __syncthreads();
+      // tile kt+1 in buf1, kt+2 in set 1, kt+3 in set 0
+      ktile_any<C, OA, OB>(buf1, buf1 + BOFF, acc);
+      if (kt + 2 < ntiles) {
+        s.template store<1>(buf0);
+        if (kt + 4 < ntiles) s.template load<1>(kt + 4);
+      }
+      __syncthreads();
+    }
   }
   if (kt < ntiles) {  // odd count: the last tile is in buf0
     ktile_any<C, OA, OB>(buf0, buf0 + BOFF, acc);

@@ -230,33 +230,22 @@ __device__ __forceinline__ void frags(const char* la, bf16x8 (&a)[C::WM][3], bf1
   }
 }
 
-// Whether a wave has the registers for a second accumulator, `low`, of the
-// five products that hold a remainder: they are 2^-8 of the result, so what
-// the matrix core cuts from their sum is too, and the leading products'
-// accumulator is cut once per k-tile and not six times (weight gradient of a
-// 1001 x 785 -> 515 layer against float64 1.55e-7 -> 1.29e-7; no time).  With
-// it the waves of 64 x 64 spill inside the k loop (8192 x 512 x 2048 103 ->
-// 181 us).
-template <class C>
-constexpr bool low_sums() { return C::WM * C::WN <= 2; }
-
 template <class C>
 __device__ __forceinline__ void mfmas(const bf16x8 (&a)[C::WM][3], const bf16x8 (&b)[C::WN][3],
-                                      f32x16 (&acc)[C::WM][C::WN], f32x16 (&low)[C::WM][C::WN]) {
-  auto term = [&](int x, int y, f32x16 (&to)[C::WM][C::WN]) {
+                                      f32x16 (&acc)[C::WM][C::WN]) {
+  auto term = [&](int x, int y) {
 #pragma unroll
     for (int i = 0; i < C::WM; ++i)
 #pragma unroll
       for (int j = 0; j < C::WN; ++j)
-        to[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][x], b[j][y], to[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i][x], b[j][y], acc[i][j], 0, 0, 0);
   };
-  f32x16(&rest)[C::WM][C::WN] = low_sums<C>() ? low : acc;
-  term(2, 0, rest);
-  term(0, 2, rest);
-  term(1, 1, rest);
-  term(1, 0, rest);
-  term(0, 1, rest);
-  term(0, 0, acc);
+  term(2, 0);
+  term(0, 2);
+  term(1, 1);
+  term(1, 0);
+  term(0, 1);
+  term(0, 0);
 }
 
 template <class C>
@@ -343,8 +332,8 @@ struct Tile {
     const int tail = left != 0 && (total - 1) % C::WGK == kg ? (total - 1) / C::WGK : -1;  // it, if mine
 
     // k-tiles in flight in registers: one where a round lasts longer than a
-    // load (256 x 256: 2.2 us), two in the short rounds of the smaller tiles
-    // (128 x 128: 0.84 -> 0.73 us a round), one where two blocks share a CU
+    // load (256 x 256: 2.2 us), two in the short rounds of the 128 x 128 tile
+    // (0.84 -> 0.73 us a round)
     f32x4 v0[4], v1[4];
     auto load = [&](int t, f32x4 (&v)[4]) {
       if (!doA && !doB) return;
@@ -375,15 +364,13 @@ struct Tile {
     const int lane = threadIdx.x & 63, h = lane >> 5, r = lane & 31;
     const int ra = wm * (C::WM * 32) + r, rb = wn * (C::WN * 32) + r;
 
-    constexpr int PF = C::WM * C::WN == 2 || C::WM * C::WN == 4 ? 2 : 1;
-    f32x16 low[C::WM][C::WN];
-    kp::zero_acc<C>(low);
+    constexpr int PF = C::WM * C::WN == 4 ? 2 : 1;
     // one round: v holds k-tile t + 1
     auto round = [&](int t, f32x4 (&v)[4]) {
       bf16x8 a[C::WM][3], b[C::WN][3];
       // the fragment reads go first where registers allow: they arrive while
       // the next k-tile is split
-      constexpr bool kReadsFirst = C::WM * C::WN == 2 || C::WM * C::WN == 4;
+      constexpr bool kReadsFirst = C::WM * C::WN == 4;
       if (kReadsFirst && t < mine) frags<C, OA, OB>(buf + (t & 1) * SB, a, b, ra, rb, h);
       if (t + 1 < mine) {
         store(t + 1, v);
@@ -395,7 +382,7 @@ struct Tile {
       __builtin_amdgcn_sched_barrier(0);
       if (t < mine) {
         __builtin_amdgcn_s_setprio(1);
-        mfmas<C>(a, b, acc, low);
+        mfmas<C>(a, b, acc);
         __builtin_amdgcn_s_setprio(0);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -419,12 +406,6 @@ struct Tile {
       if (t < nt) round(t, v1);
     }
     if (!grp) __syncthreads();
-    if constexpr (low_sums<C>()) {
-#pragma unroll
-      for (int i = 0; i < C::WM; ++i)
-#pragma unroll
-        for (int j = 0; j < C::WN; ++j) acc[i][j] += low[i][j];
-    }
     return __syncthreads_or(range.lo < kLossyCode);
   }
 
@@ -551,7 +532,7 @@ struct Tile {
   __device__ __forceinline__ static void fp32(const float* A, int64_t lda, const float* B, int64_t ldb, int64_t M,
                                            int64_t N, int64_t m0, int64_t n0, int64_t k_begin, int64_t k_end,
                                            f32x16 (&acc)[C::WM][C::WN]) {
-    constexpr int D = C::WM * C::WN >= 8 ? 1 : C::WM * C::WN == 4 ? 2 : 4;  // steps of a stage
+    constexpr int D = C::WM * C::WN >= 8 ? 1 : 2;  // steps of a stage
     struct Stage {
       f32x4 a[D][C::WM], b[D][C::WN];
     };

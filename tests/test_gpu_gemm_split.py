@@ -21,8 +21,8 @@ def operand(gen, trans, rows, k, pad, off):
     return x, m, ld
 
 
-# (M, N, K, batch): 64 x 64, 128 x 64, 128 x 128 tiles with and without
-# split-K, then 256 x 256 tiles (whole, with edges, split over K)
+# (M, N, K, batch): the fp32 64 x 64 tile with and without split-K, 128 x 128
+# and 256 x 256 tiles (whole, with edges, split over K)
 SHAPES = [(65, 63, 700, 1), (100, 515, 2000, 1), (257, 129, 33, 40), (1001, 515, 785, 1), (2000, 130, 70, 1),
           (8192, 512, 512, 1), (515, 517, 8191, 1), (256, 250, 500, 32), (4096, 4096, 2048, 1), (4090, 4087, 2051, 1),
           (1024, 4096, 4096, 1)]
