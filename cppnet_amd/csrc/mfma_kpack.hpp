@@ -93,8 +93,11 @@ struct Operand {
 
   // FAST: the whole tile is in range and 16-byte aligned.  Otherwise a unit
   // in range is one float4 load at any alignment, and the elements of the
-  // others are bounds-checked (rows < Rtot, k < Kend) and zero-filled.
-  template <bool FAST>
+  // others are bounds-checked (rows < Rtot, k < Kend) and zero-filled.  The test
+  // puts each unit's loads behind a branch of its own, one waited for after the
+  // other, so a tile of few rows (!KC), which has next to no unit in range, is
+  // read by elements alone (WIDE false).
+  template <bool FAST, bool WIDE = true>
   __device__ __forceinline__ static void load(const float* __restrict__ X, int64_t ld, int64_t r0,
                                               int64_t k0, int64_t Rtot, int64_t Kend,
                                               f32x4 (&v)[REGS]) {
@@ -107,7 +110,7 @@ struct Operand {
         v[p] = *reinterpret_cast<const f32x4*>(X + (KC ? gk + ld * gr : gr + ld * gk));
       } else {
         f32x4 t;
-        if (KC ? (gr < Rtot && gk + 3 < Kend) : (gr + 3 < Rtot && gk < Kend)) {
+        if (WIDE && (KC ? (gr < Rtot && gk + 3 < Kend) : (gr + 3 < Rtot && gk < Kend))) {
           v[p] = *reinterpret_cast<const f32x4u*>(X + (KC ? gk + ld * gr : gr + ld * gk));
           continue;
         }

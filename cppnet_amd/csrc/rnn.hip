@@ -128,7 +128,8 @@ using kp::f32x4;
 using LstmFwdCfg = kp::Cfg<1, 1, 1, 1, 16, 4>;
 constexpr int kLstmUnits = 8;  // hidden units per tile
 
-template <class LstmCfg, bool FAST>
+// FAST, WIDE: as kp::Operand::load's.
+template <class LstmCfg, bool FAST, bool WIDE>
 struct LstmFwdStage {
   using OA = kp::Operand<false, 32, LstmCfg::NT, LstmCfg::KT>;  // h(b, k) = Y[b + B(t-1) + BS k]
   using OB = kp::Operand<true, 32, LstmCfg::NT, LstmCfg::KT>;   // W_hh(k, col(n)), k-contiguous
@@ -144,7 +145,7 @@ struct LstmFwdStage {
   template <int S>
   __device__ __forceinline__ void load(int t) {
     const int64_t k0 = (int64_t)t * LstmCfg::KT;
-    OA::template load<FAST>(A, BS, b0, k0, B, H, ra[S]);
+    OA::template load<FAST, WIDE>(A, BS, b0, k0, B, H, ra[S]);
 #pragma unroll
     for (int p = 0; p < OB::PER; ++p) {
       int r, k;
@@ -169,12 +170,12 @@ struct LstmFwdStage {
   }
 };
 
-template <class LstmCfg, bool FAST>
+template <class LstmCfg, bool FAST, bool WIDE>
 __global__ void __launch_bounds__(LstmCfg::NT) lstm_step_fwd_kernel(
     float* __restrict__ gates, const float* __restrict__ bias, float* __restrict__ c,
     float* __restrict__ tanh_c, float* __restrict__ Y, const float* __restrict__ W_hh, int64_t B,
     int64_t S, int64_t H, int64_t t) {
-  constexpr int FLOATS = 2 * kp::stage_floats<LstmFwdStage<LstmCfg, FAST>>();
+  constexpr int FLOATS = 2 * kp::stage_floats<LstmFwdStage<LstmCfg, FAST, WIDE>>();
   static_assert((LstmCfg::WGK - 1) * 1024 <= FLOATS, "reduce_wgk needs more LDS");
   __shared__ __align__(16) float lds[FLOATS];
   __shared__ float tile[32 * 33];  // [col][row], padded
@@ -185,7 +186,7 @@ __global__ void __launch_bounds__(LstmCfg::NT) lstm_step_fwd_kernel(
   const int64_t j0 = (ti / nbt) * kLstmUnits;
   kp::f32x16 acc[1][1];
   kp::zero_acc<LstmCfg>(acc);
-  LstmFwdStage<LstmCfg, FAST> s(Y + B * (t - 1), W_hh, BS, B, H, b0, j0);
+  LstmFwdStage<LstmCfg, FAST, WIDE> s(Y + B * (t - 1), W_hh, BS, B, H, b0, j0);
   kp::pipeline<LstmCfg>((int)((H + LstmCfg::KT - 1) / LstmCfg::KT), lds, s, acc);
   kp::reduce_wgk<LstmCfg>(lds, acc);
   kp::for_each_acc_run<LstmCfg>(acc, [&](int ml, int nl, const kp::f32x4& v) {
@@ -1642,7 +1643,11 @@ int lstm_fwd_steps(float* gates, const float* b, float* c, float* tanh_c, float*
   // FAST: full tiles, whole k-tiles, 16-byte aligned rows of Y and W_hh
   const bool fast = B % 32 == 0 && H % Cfg::KT == 0 && H % kLstmUnits == 0 && (B * S) % 4 == 0 &&
                     aligned16(Y) && aligned16(W_hh);
-  const auto kern = fast ? &lstm_step_fwd_kernel<Cfg, true> : &lstm_step_fwd_kernel<Cfg, false>;
+  // fewer than 16 samples, half of a tile: by elements (one sample, H 512: 13.4
+  // us a step against 16.8; 200 samples 17 against 15)
+  const auto kern = fast      ? &lstm_step_fwd_kernel<Cfg, true, true>
+                    : B >= 16 ? &lstm_step_fwd_kernel<Cfg, false, true>
+                              : &lstm_step_fwd_kernel<Cfg, false, false>;
   for (int64_t t = 1; t < S; ++t) {
     TimingRec* rec = timing_slot(2.0 * B * 4 * H * H);
     if (rec) (void)hipEventRecord(rec->start, st);
