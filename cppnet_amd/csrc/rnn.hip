@@ -339,10 +339,18 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));  // two (value bits,
 // Each 8-byte word lies inside the one store, so a reader never sees a value
 // without its stamp; the store covers half as many cache-line pieces per
 // instruction as two 8-byte stores.
+// A store of more than 8 bytes reads its data registers after it has issued:
+// they must not be written in the next two wait states.  The compiler sees to
+// that only where the store has no scalar offset, and so wrote the next pair
+// over this one at once; with a second wave on the SIMD the wrong value went
+// out under a right stamp (gradients off by 1-2% wherever a CU held two
+// blocks: B 1600, H 64 and up).  The empty use of v keeps its registers until
+// the s_nop is over.
 __device__ __forceinline__ void ex_store_pair(__amdgpu_buffer_rsrc_t rs, unsigned voff, unsigned soff, float a,
                                               float b, unsigned stamp) {
   const u32x4 v = {__float_as_uint(a), stamp, __float_as_uint(b), stamp};
   __builtin_amdgcn_raw_buffer_store_b128(v, rs, voff, soff, 1);
+  asm volatile("s_nop 1" ::"v"(v) : "memory");
 }
 
 // Raw buffer resource over the exchange area (32-bit byte offsets).

@@ -9,7 +9,9 @@ from cppnet_amd import ops
 pytestmark = pytest.mark.gpu
 
 CASES = [(1, 2, 3, 1), (3, 5, 4, 8), (17, 6, 64, 64), (16, 4, 5, 65), (40, 6, 12, 71), (33, 5, 7, 129), (130, 3, 9, 300),
-         (5, 9, 16, 511), (100, 4, 128, 256), (120, 3, 8, 512)]
+         (5, 9, 16, 511), (100, 4, 128, 256), (120, 3, 8, 512),
+         # multiples of 16 and tuned hidden sizes: two and more blocks a CU
+         (1600, 3, 5, 64), (4000, 3, 5, 64), (2000, 3, 5, 128), (1600, 3, 64, 64)]
 
 
 @pytest.mark.parametrize("B,S,I,H", CASES)
