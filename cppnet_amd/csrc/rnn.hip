@@ -2152,9 +2152,24 @@ int gru_persistent(bool fwd, GruPersistArgs args, int64_t B, int64_t S, int64_t 
   return CNHIP_OK;
 }
 
+// Steps from which the any-size persistent LSTM is the faster form.  It loads
+// its share of W_hh into registers and waits for the chip's blocks once, a
+// per-step launch (which needs no exchange) costs 4-15 us a step.  Measured
+// with the layer's GEMMs over H 16 .. 512, B 1 .. 4001 and 2 to 20 steps, time
+// against the per-step launches': forward with up to 128 blocks of H <= 128
+// 0.91-1.2 at 2 steps, 0.77-0.95 at 3; up to 256 blocks 0.85-1.06 at 3,
+// 0.70-0.91 at 4; 512 blocks 1.02 at 4, 0.74-0.91 at 6; more 0.87-1.12 at 6,
+// 0.75-0.99 at 10.  Backward, whose blocks gather four gate gradients, H <= 128
+// 0.87-1.07 at 4, 0.84-1.04 at 6; H <= 256 1.0-1.15 at 6, 0.86-1.04 at 16; above
+// 0.95-1.16 at 4, 0.79-0.98 at 10.  (The GRU's is the faster one from 2 steps.)
+int64_t lstm_any_min_steps(bool fwd, int64_t H, int64_t grid) {
+  if (!fwd) return H <= 128 ? 6 : H <= 256 ? 16 : 8;
+  return grid <= 128 && H <= 128 ? 3 : grid <= 256 ? 4 : grid <= 512 ? 6 : 10;
+}
+
 // The LSTM recurrence (forward or BPTT) of any B and any H up to 512 in one
-// persistent launch, where the chip holds its blocks; false in *done to fall
-// back to the per-step launches.
+// persistent launch, where the chip holds its blocks and it is the faster form
+// (lstm_any_min_steps); false in *done to fall back to the per-step launches.
 template <int HP>
 const void* lstm_any_kernel(bool fwd) {
   return fwd ? reinterpret_cast<const void*>(&lstm_fwd_any_kernel<HP>)
@@ -2170,6 +2185,7 @@ int lstm_any_persistent(bool fwd, LstmAnyArgs args, int64_t B, int64_t S, int64_
                                 : lstm_any_kernel<512>(fwd);
   const int64_t nst = (B + kPt - 1) / kPt, nut = (H + kPt - 1) / kPt, grid = 8 * nut * ((nst + 7) / 8);
   const size_t ex_bytes = (size_t)(fwd ? 2 : 8) * nst * nut * kPt * kPt * sizeof(u64);
+  if (S < lstm_any_min_steps(fwd, H, grid)) return CNHIP_OK;
   if (ex_bytes > 0x7fffffffu || !persist_fits(kern, grid, 256, who)) return CNHIP_OK;
   args.B = (int)B;
   args.S = (int)S;

@@ -1,10 +1,12 @@
 """The persistent LSTM recurrence for batches and hidden sizes that are no
 multiple of 16 against float64, at the edges of its tiles and each padded
 width, with gradients of every step and of the last one only."""
+import ctypes
+
 import pytest
 import torch
 
-from cppnet_amd import ops
+from cppnet_amd import _capi, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +67,48 @@ def test_lstm_any_matches_float64(gpu, monkeypatch, B, S, I, H, last, path):
         assert rel <= lim, f"{name}: {rel:.3g} > {lim:.3g}"
     for a, w in zip(got, run()):
         assert torch.equal(a, w), "two runs differ"
+
+
+def recurrence_launches(fn):
+    """MFMA launches of fn (its GEMMs and the recurrence's)."""
+    lib = _capi.load()
+    n, ms, fl = ctypes.c_int64(), ctypes.c_double(), ctypes.c_double()
+    _capi.check(lib.cnhip_gemm_timing_enable(1))
+    try:
+        fn()
+        _capi.check(lib.cnhip_gemm_timing_read(ctypes.byref(n), ctypes.byref(ms), ctypes.byref(fl)))
+    finally:
+        _capi.check(lib.cnhip_gemm_timing_enable(0))
+    return n.value
+
+
+# (B, S, H, whether forward / backward run in one launch).  Few steps are faster
+# step by step; two sample tiles an XCD (B > 128) fit beside each other at H <=
+# 256, where the backward needs less than half of a CU's LDS, and not at 300
+@pytest.mark.parametrize("B,S,H,fwd,bwd", [(17, 2, 65, False, False), (17, 3, 65, True, False), (17, 6, 65, True, True),
+                                           (100, 3, 256, False, False), (100, 16, 256, True, True), (5, 8, 511, True, True),
+                                           (200, 6, 100, True, True), (250, 16, 200, True, True), (130, 16, 300, False, False),
+                                           (4001, 6, 64, False, True), (4001, 10, 64, True, True)])
+def test_lstm_any_path(gpu, monkeypatch, B, S, H, fwd, bwd):
+    I = 8
+    gen = torch.Generator("cuda").manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=gen, device="cuda")  # noqa: E731
+    X, Wi, Wh, b, dY = r(I, S, B), r(4 * H, I) / 4, r(4 * H, H) / (2 * H) ** 0.5, r(4 * H) / 10, r(H, S, B) / B
+    e = lambda *s: torch.empty(*s, device="cuda")  # noqa: E731
+    out = {}
+    for path in ("1", "0"):
+        monkeypatch.setenv("CNHIP_RECURRENCE_PERSISTENT", path)
+        Y, gates, c, tc, gWi, gWh, gb, dX = (e(H, S, B), e(4 * H, S, B), e(H, S, B), e(H, S, B), e(4 * H, I), e(4 * H, H),
+                                             e(4 * H), e(I, S, B))
+        nf = recurrence_launches(lambda: ops.lstm_forward(X, Wi, Wh, b, Y, gates, c, tc, B, S, I, H))
+        nb = recurrence_launches(
+            lambda: ops.lstm_backward(X, Wi, Wh, Y, gates, c, tc, dY, gWi, gWh, gb, dX, B, S, I, H))
+        out[path] = (nf, nb, Y, gates, c, gWi, gWh, gb, dX)
+    (nf, nb, *got), (sf, sb, *want) = out["1"], out["0"]
+    # one launch in place of S - 1; the rest of both passes is the same
+    assert sf - nf == (S - 2 if fwd else 0), (sf, nf)
+    assert sb - nb == (S - 2 if bwd else 0), (sb, nb)
+    for g, w in zip(got, want):
+        # two fp32 forms of sums of at most max(B S, 4 H) terms through S steps
+        lim = 16 * 2.0 ** -24 * max(B * S, 4 * H) ** 0.5 * S ** 0.5 + 1e-6
+        assert float((g - w).norm()) <= lim * float(w.norm()) + 1e-30
