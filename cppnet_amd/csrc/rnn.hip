@@ -1935,8 +1935,12 @@ unsigned persist_epoch(int dev, uint64_t gen, bool capturing, bool* zero, int* s
   return e.next++;
 }
 
-// Zeroes the fault word, the XCD slot counters and the exchange area
-// (ex_bytes, after a 256-byte header) where persist_epoch asks for it, then
+// Zeroes the fault word, the XCD slot counters and the exchange area (after a
+// 256-byte header) where persist_epoch asks for it, the whole allocation and
+// not only this launch's ex_bytes: a later, larger launch finds the allocation
+// marked clean and must not poll words that never were zeroed (a GRU's forward
+// exchanges 4 areas, its backward 6).  A captured launch zeroes its own words
+// before each replay.  Then
 // launches `kernel` with one argument (cooperatively only when asked to
 // above, and never while the stream is being captured into a graph).
 // Header words: 0 the fault word, 16 + 8 k the counter set k (k = 0, 1, 2).
@@ -1946,7 +1950,8 @@ int persist_launch(const void* kernel, int64_t grid, int threads, Args& args, si
   void* ws = nullptr;
   uint64_t gen = 0;
   const size_t bytes = 256 + ex_bytes;
-  CNHIP_TRY(scratch(st, kScratchRecur, bytes, &ws, &gen, who));
+  size_t cap = 0;
+  CNHIP_TRY(scratch(st, kScratchRecur, bytes, &ws, &gen, &cap, who));
   int dev = 0;
   CNHIP_TRY(check_hip(hipGetDevice(&dev), who));
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -1967,7 +1972,7 @@ int persist_launch(const void* kernel, int64_t grid, int threads, Args& args, si
     args.sync.epoch = persist_epoch(dev, gen, capturing, &zero, &set);
     args.sync.slots = head + 16 + 8 * set;
     args.sync.slots_next = set == 2 ? nullptr : head + 16 + 8 * (1 - set);
-    if (zero) CNHIP_TRY(fill_bytes(ws, 0, bytes, st, who));
+    if (zero) CNHIP_TRY(fill_bytes(ws, 0, capturing ? bytes : cap, st, who));
     if (!capturing && persist_cooperative())
       CNHIP_TRY(check_hip(hipLaunchCooperativeKernel(kernel, dim3((unsigned)grid), dim3(threads), params, 0, st), who));
     else

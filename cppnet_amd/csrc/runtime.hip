@@ -133,10 +133,10 @@ int persist_order_leave(hipStream_t stream, int dev, const char* who) {
 }
 
 int scratch(hipStream_t stream, int slot, size_t bytes, void** ptr, const char* where) {
-  return scratch(stream, slot, bytes, ptr, nullptr, where);
+  return scratch(stream, slot, bytes, ptr, nullptr, nullptr, where);
 }
 
-int scratch(hipStream_t stream, int slot, size_t bytes, void** ptr, uint64_t* gen, const char* where) {
+int scratch(hipStream_t stream, int slot, size_t bytes, void** ptr, uint64_t* gen, size_t* cap_out, const char* where) {
   if (t_fixed.p) {
     if (slot != kScratchGemm) {
       set_error("%s: scratch slot %d requested inside a no-allocation call", where, slot);
@@ -149,6 +149,7 @@ int scratch(hipStream_t stream, int slot, size_t bytes, void** ptr, uint64_t* ge
     }
     *ptr = t_fixed.p;
     if (gen) *gen = 0;
+    if (cap_out) *cap_out = t_fixed.cap;
     return CNHIP_OK;
   }
   int dev = 0;
@@ -185,6 +186,7 @@ int scratch(hipStream_t stream, int slot, size_t bytes, void** ptr, uint64_t* ge
   }
   *ptr = e->p;
   if (gen) *gen = e->gen;
+  if (cap_out) *cap_out = e->cap;
   return CNHIP_OK;
 }
 

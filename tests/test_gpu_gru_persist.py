@@ -89,3 +89,30 @@ def test_gru_fault_is_reported_and_taken(gpu, monkeypatch):
     got = run(t, B, S, I, H)
     for k in want:
         assert torch.equal(got[k], want[k]), k
+
+
+def test_exchange_area_is_zeroed_whole(gpu):
+    """The first recurrent launch in a stream's exchange buffer zeroes all of
+    it, so that the larger exchange of a later launch in the same allocation
+    (the backward's) never reads words that were not zeroed."""
+    B, S, I, H = 32, 4, 8, 64
+    t = tensors(B, S, I, H, 5)
+    lib = _capi.load()
+
+    def filled(fn):
+        _capi.check(lib.cnhip_hbm_timing_enable(1))
+        try:
+            fn()
+            return sum(r["total_bytes"] for r in _capi.hbm_timing_rows() if r["kernel"] == "fill_bytes_kernel")
+        finally:
+            _capi.check(lib.cnhip_hbm_timing_enable(0))
+
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        first = filled(lambda: ops.gru_forward(t["X"], t["Wi"], t["Wh"], t["b"], t["Y"], t["gates"], t["rh"], B, S, I, H))
+        later = filled(lambda: ops.gru_backward(t["X"], t["Wi"], t["Wh"], t["Y"], t["gates"], t["rh"], t["dY"], t["gWi"],
+                                                t["gWh"], t["gb"], t["dX"], B, S, I, H))
+        torch.cuda.synchronize()
+    need = 256 + 6 * B * H * 8  # the backward's six areas of 8-byte words
+    assert later == 0, "the exchange buffer was grown or zeroed again: not the case that is tested"
+    assert first >= need, f"zeroed {first} bytes, the backward polls up to {need}"
