@@ -201,9 +201,11 @@ __global__ void __launch_bounds__(C::NT) conv_pixel_kernel(ConvArgs a) {
   // (tap ascending), and its tables map contraction index j OC + oc (j: the
   // listed tap) to the element of dY and the row of W'.  Stride 2, 5 x 5, 100
   // samples x 17 x 29 x 27: 94 -> 40 us against all 1000 contraction indices.
+  // A 1 x 1 filter has one tap to list, which costs more than it saves (256
+  // samples x 64 x 8 x 8 to 128, stride 2, backward 28 us without, 31 with).
   __shared__ uint16_t wtbl[TBL && DGRAD ? KTBL : 4];
   __shared__ int taps;
-  const bool listed = TBL && DGRAD && d.S > 1;
+  const bool listed = TBL && DGRAD && d.S > 1 && d.KS > 1;
   if (listed) {
     const int OC = (int)d.OC, T = (int)(d.KS * d.KS);
     if (threadIdx.x < 64) {
