@@ -82,3 +82,14 @@ def test_plans_do_not_depend_on_what_was_planned_before():
         M, N, K, b, ta, tb = jobs[i]
         assert plan(M, N, K, b, ta, tb) == first[i]
         plan(M, N, K, b, ta, tb, reads_c=True)
+
+
+# What tests/test_gpu_gemm_split.py is to reach: (M, N, K), tile, splits
+@pytest.mark.parametrize("size,tile,splits", [((100, 515, 2000), 64, 21), ((1001, 515, 785), 64, 5), ((8192, 512, 512), 128, 1),
+                                              ((2050, 1561, 425), 128, 1), ((196, 2287, 3134), 128, 7),
+                                              ((2048, 2048, 512), 128, 1), ((4096, 4096, 2048), 256, 1),
+                                              ((4090, 4087, 2051), 256, 1), ((6731, 586, 2027), 256, 2),
+                                              ((4057, 257, 5017), 256, 8), ((1361, 385, 8687), 256, 16)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+def test_the_gpu_tests_reach_every_tile(size, tile, splits, ta, tb):
+    assert plan(*size, 1, ta, tb)[:3] == (tile, tile, splits)

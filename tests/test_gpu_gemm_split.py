@@ -1,7 +1,7 @@
 """The GEMM shapes that run on the bf16 matrix cores with operands split in
-three: tile edges, remainders of K, odd leading dimensions and unaligned
-operands, every orientation and tile shape, against float64; and what bf16
-terms cannot hold (infinities, NaN, values near the ends of the fp32 range),
+three, and the fp32 tile beside them: tile edges, remainders of K, odd leading
+dimensions and unaligned operands, every orientation and tile shape, against
+float64; and what bf16 terms cannot hold (infinities, NaN, values near the ends of the fp32 range),
 against IEEE fp32 semantics."""
 import numpy as np
 import pytest
@@ -22,10 +22,12 @@ def operand(gen, trans, rows, k, pad, off):
 
 
 # (M, N, K, batch): the fp32 64 x 64 tile with and without split-K, 128 x 128
-# and 256 x 256 tiles (whole, with edges, split over K)
+# tiles whole and ragged, and 256 x 256 tiles whole, with edges, and with edges and a ragged K
+# in 2, 8 and 16 splits (tests/test_gemm_plan.py asserts which runs where)
 SHAPES = [(65, 63, 700, 1), (100, 515, 2000, 1), (257, 129, 33, 40), (1001, 515, 785, 1), (2000, 130, 70, 1),
           (8192, 512, 512, 1), (515, 517, 8191, 1), (256, 250, 500, 32), (4096, 4096, 2048, 1), (4090, 4087, 2051, 1),
-          (1024, 4096, 4096, 1)]
+          (1024, 4096, 4096, 1), (2050, 1561, 425, 1), (196, 2287, 3134, 1), (6731, 586, 2027, 1), (4057, 257, 5017, 1),
+          (1361, 385, 8687, 1)]
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
@@ -63,7 +65,7 @@ def test_gemm_split_matches_float64(gpu, ta, tb, M, N, K, batch):
     assert abs(float((got - want).mean())) <= (6 / (M * N * batch) ** 0.5 + 0.02) * 2.0 ** -24 * (K / 2) ** 0.5 * rms
 
 
-@pytest.mark.parametrize("M,N,K", [(64, 80, 700), (1001, 515, 785), (4096, 4096, 2048)])
+@pytest.mark.parametrize("M,N,K", [(64, 80, 700), (1001, 515, 785), (196, 2287, 3134), (2048, 2048, 512), (4096, 4096, 2048)])
 def test_gemm_split_nonfinite_and_range_ends(gpu, M, N, K):
     gen = torch.Generator("cuda").manual_seed(K)
     A = torch.randn(K, M, generator=gen, device="cuda")  # A(m, k) at [k, m]
@@ -136,7 +138,8 @@ def low_end(A, B, case):
                                   ("all", -100, -36), ("row", -140, 100), ("row", -120, 20), ("cross", -66, -66),
                                   ("cross", -70, -72)], ids=str)
 @pytest.mark.parametrize("sign", ["mixed", "one"])
-@pytest.mark.parametrize("M,N,K", [(65, 80, 700), (300, 515, 785), (4096, 4096, 2048)])
+@pytest.mark.parametrize("M,N,K", [(65, 80, 700), (300, 515, 785), (196, 2287, 3134), (2048, 2048, 512),
+                                   (4096, 4096, 2048)])
 def test_gemm_split_low_end_of_the_range(gpu, M, N, K, case, sign):
     """Operands whose low bits, or all of them, lie below the bf16 terms' grid,
     and products that are subnormal."""
