@@ -509,7 +509,7 @@ int cnhip_linear_backward(const float* X, const float* W, const float* dY, float
                                   beta, grad_W, in_features, 0, 1, nullptr, CNHIP_EPI_NONE, nullptr,
                                   nullptr, 0};
       if (dX) {
-        // dX and dW in one launch where their tiles leave half the chip's block slots empty
+        // dX and dW in one launch where both take the same split-operand tile and dX does not split K
         const cnhip::GemmSpec dgrad{0, 1, batch, in_features, out_features, 1.f, dY, batch, 0, W,
                                     in_features, 0, 0.f, dX, batch, 0, 1, nullptr, CNHIP_EPI_NONE,
                                     nullptr, nullptr, 0};
@@ -580,7 +580,7 @@ int cnhip_linear_backward_act(const float* X, const float* W, const float* dY, f
     CNHIP_TRY(cnhip::linear_wgrad_small(X, dY, grad_W, grad_b, batch, in_features, out_features, accumulate,
                                         st, who, &fused));
     if (!fused) {
-      // dX and dW in one launch where their tiles leave half the chip's block slots empty
+      // dX and dW in one launch where both take the same split-operand tile and dX does not split K
       const cnhip::GemmSpec wgrad{1, 0, in_features, out_features, batch, 1.f, X, batch, 0, dY, batch, 0,
                                   accumulate ? 1.f : 0.f, grad_W, in_features, 0, 1, nullptr,
                                   CNHIP_EPI_NONE, nullptr, nullptr, 0};
