@@ -656,8 +656,8 @@ constexpr int64_t kMaxPartialBytes = (int64_t)32 << 20;
 // pipes need.  Fitted to sweeps of every shape and split count over 113 sizes
 // in the three orientations of a layer (64^3 to 4096^3 and 8192 x 2048 x 512,
 // ragged ones, batches up to 512, contractions up to 60000): the plan takes
-// 0.9% longer than the best of them in the mean, 30% at worst (2000^3, where
-// 256 x 256 tiles in two splits beat their edges' cost).
+// 0.9% longer than the best of them in the mean, 15% at worst but for 2000^3
+// (30%: 256 x 256 tiles in two splits beat their edges' cost).
 struct ShapeCost {
   int64_t slots;
   double t_round, t_lat, t_tile;
@@ -665,9 +665,9 @@ struct ShapeCost {
 
 ShapeCost shape_cost(Shape shape) {
   switch (shape) {
-    case Shape::XX: return {256, 10.6e-6, 0, 3.53e-6};
-    case Shape::M: return {256, 5.31e-6, 0, 1.42e-6};
-    case Shape::S: return {1024, 2.0e-6, 1.31e-6, 0.501e-6};
+    case Shape::XX: return {256, 10.8e-6, 0, 2.89e-6};
+    case Shape::M: return {256, 4.0e-6, 0, 1.38e-6};
+    case Shape::S: return {1024, 1.6e-6, 1.1e-6, 0.496e-6};
     case Shape::SN: return {1024, 0, 2.0 * CfgSN::BM * CfgSN::BN * KQ / (157.3e12 / 256) * 4 / 0.8, 0};
     case Shape::SM: return {1024, 0, 2.0 * CfgSM::BM * CfgSM::BN * KQ / (157.3e12 / 256) * 4 / 0.8, 0};
   }
@@ -679,7 +679,7 @@ ShapeCost shape_cost(Shape shape) {
 // for it the whole product takes longer: by kSplitEdge and kEdge, and for the
 // split shapes kSplitTail more where K is no multiple of the k-tile (8102 x
 // 613 x 4079: 610 us, the 64 x 64 tile 395).
-constexpr double kSplitEdge = 1.45, kSplitTail = 1.06, kEdge = 1.21;
+constexpr double kSplitEdge = 1.45, kSplitTail = 1.12, kEdge = 1.3;
 
 int64_t shape_tiles(Shape shape, int64_t M, int64_t N) {
   switch (shape) {
@@ -732,7 +732,11 @@ double split_cost(Shape shape, int64_t M, int64_t N, int64_t K, int64_t batches,
   shape_tile(shape, &tm, &tn);
   const bool split = shape == Shape::XX || shape == Shape::M;
   double t_tile = c.t_tile;
-  if (!skinny && (M % tm != 0 || N % tn != 0 || K % sp::KT != 0)) t_tile *= split ? kSplitEdge : kEdge;
+  double t_lat = c.t_lat;
+  if (!skinny && (M % tm != 0 || N % tn != 0 || K % sp::KT != 0)) {
+    t_tile *= split ? kSplitEdge : kEdge;
+    t_lat *= kEdge;
+  }
   if (split && K % sp::KT != 0) t_tile *= kSplitTail;
   double best = INFINITY;
   splits = 1;
@@ -745,8 +749,8 @@ double split_cost(Shape shape, int64_t M, int64_t N, int64_t K, int64_t batches,
       if (n == 1 ? !can_park : n % 2 != 0) continue;
     }
     const double kt = (double)(kps / KQ), rounds = (double)((blocks * s + c.slots - 1) / c.slots);
-    double cost = rounds * c.t_round + kt * std::max(rounds * c.t_lat, (double)((blocks * s + 255) / 256) * t_tile);
-    if (s > 1) cost += (double)(s + 1) * M * N * batches * 4.0 / 5.2e12 + 3.2e-6;
+    double cost = rounds * c.t_round + kt * std::max(rounds * t_lat, (double)((blocks * s + 255) / 256) * t_tile);
+    if (s > 1) cost += (double)(s + 1) * M * N * batches * 4.0 / 3.1e12 + 3.5e-6;
     if (cost < best) {
       best = cost;
       splits = (int)s;
