@@ -133,8 +133,9 @@ CPU_LOOPS_BATCH = {1: 512, 2: 64}
 # rocprofv3 PMC runs (FETCH_SIZE, WRITE_SIZE) of that config scaled by a
 # reference kernel of known traffic (bench.py --traffic-calibration),
 # averaged over the class's launches of a step; the runs, the factors and the
-# per-kernel tables are in profiles/*_counters.md.
-PMC_TRAFFIC_BYTES = {1: 0.6e6, 2: 471.9e6, 3: 39.3e6, 4: 955.1e6, 5: 170.4e6}
+# per-kernel tables are in profiles/*_counters.md (configs 3 and 4: their
+# convolutions and recurrence; their few GEMMs run in other tiles since).
+PMC_TRAFFIC_BYTES = {1: 0.6e6, 2: 682.8e6, 3: 39.3e6, 4: 955.1e6, 5: 188.8e6}
 
 
 def _cpu_model() -> str:

@@ -166,8 +166,8 @@ __device__ __forceinline__ void mfma_ktile(const float* __restrict__ la,
   const int kb = wk * C::BK + (C::BK / 2) * h;
   // Waves with 2 x 2 or more accumulator blocks raise their issue priority
   // for the k-tile's MFMAs, so a SIMD's matrix pipe is fed ahead of the other
-  // waves' staging loads (config 2's 128 x 256 tiles: 0.9% per train step,
-  // measured; the 128 x 128 tile was measured slower with it).
+  // waves' staging loads.  The convolutions' 128 x 128 tile, the only one of
+  // that size here now, runs the same with and without (48 passes, 0.1%).
   if constexpr (C::WM * C::WN >= 4) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int c = 0; c < C::BK / 8; ++c) {
